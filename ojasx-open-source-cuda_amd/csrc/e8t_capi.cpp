@@ -137,8 +137,17 @@ static int check_fmt_args(int fmt, const void* a, const uint8_t* packed, const u
 
 // Kernel family of a forward / backward launch (the dispatch below).  Pointer alignment
 // takes part in it; the workspace query passes null pointers (aligned).
-enum Route { kRouteGemvTile, kRouteGemv2m, kRouteGemv, kRouteGemv2, kRouteMfma, kRouteGeneric };
+enum Route { kRouteGemvTile, kRouteGemv2m, kRouteGemv, kRouteGemv2, kRouteMfma, kRouteF32,
+             kRouteGeneric };
 
+// fp32 activations and the shapes the 16-bit kernels do not take: the fp32 matrix
+// instruction where rows hold whole scale groups of a power of two, else (groups that cross
+// rows, group sizes like 24 or 48, 2-bit group size 4) the SIMT tiles.
+static Route general_route(const void* a, const uint8_t* packed, const uint16_t* scales,
+                           int64_t M, int64_t N, int64_t K, int64_t gs, int fmt, bool bwd) {
+    return ojx::gemm_f32_supported(a, packed, scales, M, N, K, gs, fmt, bwd) ? kRouteF32
+                                                                            : kRouteGeneric;
+}
 
 static Route route_fwd(int fmt, const void* x, const uint8_t* packed, const uint16_t* scales,
                        const void* y, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype) {
@@ -160,20 +169,20 @@ static Route route_fwd(int fmt, const void* x, const uint8_t* packed, const uint
             return kRouteGemv;
         if (M > 16 && ojx::gemm_mfma_supported(x, packed, scales, M, N, K, gs, dtype, fmt))
             return kRouteMfma;
-        return kRouteGeneric;
+        return general_route(x, packed, scales, M, N, K, gs, fmt, false);
     }
     if (ojx::gemv2_supported(x, packed, scales, y, M, N, K, gs, dtype, fmt))
         return kRouteGemv2;
     if (ojx::gemv2m_supported(x, packed, scales, y, M, N, K, gs, dtype, fmt)) return kRouteGemv2m;
     if (ojx::gemm_mfma_supported(x, packed, scales, M, N, K, gs, dtype, fmt)) return kRouteMfma;
-    return kRouteGeneric;
+    return general_route(x, packed, scales, M, N, K, gs, fmt, false);
 }
 
 static Route route_bwd(int fmt, const void* gy, const uint8_t* packed, const uint16_t* scales,
                        int64_t M, int64_t N, int64_t K, int64_t gs, int dtype) {
     if (N > 0 && ojx::gemm_mfma_supported(gy, packed, scales, M, N, K, gs, dtype, fmt, true))
         return kRouteMfma;
-    return kRouteGeneric;
+    return general_route(gy, packed, scales, M, N, K, gs, fmt, true);
 }
 
 static const char* fmt_name(int fmt) {
@@ -231,6 +240,9 @@ static int gemm_fwd(int fmt, const void* x, const uint8_t* packed, const uint16_
         e = launch_mfma(x, packed, scales, bias, y, M, N, K, gs, dtype, s, fmt, false, ws,
                         ws_bytes, lora);
         break;
+    case kRouteF32:
+        e = ojx::launch_gemm_f32_fwd(x, packed, scales, bias, y, M, N, K, gs, dtype, s, fmt, lora);
+        break;
     case kRouteGeneric:
         e = ojx::launch_gemm_generic_fwd(x, packed, scales, bias, y, M, N, K, gs, dtype, s, fmt,
                                          lora);
@@ -285,10 +297,18 @@ static int gemm_bwd(int fmt, const void* grad_y, const uint8_t* packed, const ui
     if (int r = check_device()) return r;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
-    if (route_bwd(fmt, grad_y, packed, scales, M, N, K, gs, dtype) == kRouteMfma)
+    const Route route = route_bwd(fmt, grad_y, packed, scales, M, N, K, gs, dtype);
+    if (route == kRouteMfma) {
         e = launch_mfma(grad_y, packed, scales, nullptr, grad_x, M, N, K, gs, dtype, s, fmt, true,
                         ws, ws_bytes);
-    else
+    } else if (route == kRouteF32) {
+        int splits = ojx::gemm_f32_bwd_splits(M, N, K);
+        const size_t per = (size_t)ojx::split_stride(M, K) * sizeof(float);
+        const size_t fit = ws ? ws_bytes / per : 0;
+        if ((size_t)splits > fit) splits = fit < 2 ? 1 : (int)fit;
+        e = ojx::launch_gemm_f32_bwd(grad_y, packed, scales, grad_x, static_cast<float*>(ws),
+                                     splits, M, N, K, gs, dtype, s, fmt);
+    } else
         e = ojx::launch_gemm_generic_bwd(grad_y, packed, scales, grad_x, M, N, K, gs, dtype, s,
                                          fmt);
     if (e != hipSuccess) return fail(OJX_EHIP, "%s gemm_bwd_dx launch: %s", fmt_name(fmt),
@@ -315,6 +335,9 @@ static int workspace_bytes(int fmt, int bwd, int64_t M, int64_t N, int64_t K, in
         const int64_t out_cols = bwd ? K : N, red = bwd ? N : K;
         *bytes = ojx::gemm_split_bytes(ojx::gemm_mfma_choice(M, out_cols, red, bwd != 0), M,
                                        out_cols);
+    } else if (r == kRouteF32 && bwd) {
+        *bytes = ojx::gemm_split_bytes(
+            ojx::GemmChoice{true, ojx::gemm_f32_bwd_splits(M, N, K)}, M, K);
     }
     g_last_error[0] = '\0';
     return OJX_OK;

@@ -1,9 +1,9 @@
 // e8t_gemm_generic.hip -- general LDS-tiled SIMT kernels for the fused E8 linear
 // (ternary 1.5-bit and 2-bit codes).
 //
-// These cover every shape and dtype the op accepts (fp32 activations, K not a
-// multiple of the MFMA chunk, flat layouts whose groups cross rows, as the
-// reference's portable path allows: lattice.py:613-624).  Weights are decoded
+// These cover every shape and dtype the op accepts; launched for what no other kernel
+// takes: flat layouts whose groups cross rows, as the reference's portable path allows
+// (lattice.py:613-624), group sizes that are no power of two or under 8, misaligned views.  Weights are decoded
 // per element from the flat index f = n*K + k straight into LDS, so no dense
 // weight ever reaches HBM.  fp32 accumulation; the decoded weight follows the
 // reference's dtype rule (coord * scales.to(dtype)).

@@ -1004,6 +1004,22 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
     }
 }
 
+hipError_t launch_split_reduce(const float* part, int splits, const void* bias, void* y,
+                               int64_t M, int64_t N, int dt, hipStream_t stream,
+                               const LoraEp& lora) {
+    const dim3 grid((unsigned)((M * N + 1023) / 1024));
+    if (dt == kF32)
+        hipLaunchKernelGGL((gemm_split_reduce_kernel<kF32>), grid, dim3(256), 0, stream, part,
+                           splits, bias, y, M, N, lora);
+    else if (dt == kF16)
+        hipLaunchKernelGGL((gemm_split_reduce_kernel<kF16>), grid, dim3(256), 0, stream, part,
+                           splits, bias, y, M, N, lora);
+    else
+        hipLaunchKernelGGL((gemm_split_reduce_kernel<kBF16>), grid, dim3(256), 0, stream, part,
+                           splits, bias, y, M, N, lora);
+    return hipGetLastError();
+}
+
 bool gemm_mfma_supported(const void* x, const uint8_t* packed, const uint16_t* scales,
                          int64_t M, int64_t N, int64_t K, int64_t gs, int dt, int fmt,
                          bool bwd) {
@@ -1040,12 +1056,10 @@ static hipError_t launch_cfg(const void* x, const uint8_t* packed, const uint16_
     hipLaunchKernelGGL((gemm_mfma_kernel<DT, C, FMT, GS2, BWD>), dim3((unsigned)(tiles * splits)),
                        dim3(C::THREADS), 0, stream, x, packed, scales, bias, y, part, splits, M,
                        N, K, lora);
-    if (splits == 1) return hipGetLastError();
-    const int64_t groups = (M * NO + 1023) / 1024;
-    hipLaunchKernelGGL((gemm_split_reduce_kernel<DT>), dim3((unsigned)groups), dim3(256), 0,
-                       stream, part, splits, BWD ? nullptr : bias, y, M, NO,
-                       BWD ? LoraEp{} : lora);
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    if (splits == 1 || e != hipSuccess) return e;
+    return launch_split_reduce(part, splits, BWD ? nullptr : bias, y, M, NO, DT, stream,
+                               BWD ? LoraEp{} : lora);
 }
 
 // Tile configuration and K split of a launch.

@@ -68,6 +68,27 @@ hipError_t launch_gemm_generic_bwd(const void* gy, const uint8_t* packed, const 
                                    void* gx, int64_t M, int64_t N, int64_t K, int64_t gs, int dt,
                                    hipStream_t stream, int fmt = 0);
 
+// The fused linear on the fp32 matrix instruction: every dtype, any M and N, rows of whole
+// scale groups (K % gs == 0) of 2^t >= 8 weights.  The backward's row splits (fp32 partial
+// sums, splits * split_stride(M, K) floats in `part`) come from gemm_f32_bwd_splits; fewer
+// are fine.
+bool gemm_f32_supported(const void* x, const uint8_t* packed, const uint16_t* scales, int64_t M,
+                        int64_t N, int64_t K, int64_t gs, int fmt, bool bwd);
+int gemm_f32_bwd_splits(int64_t M, int64_t N, int64_t K);
+hipError_t launch_gemm_f32_fwd(const void* x, const uint8_t* packed, const uint16_t* scales,
+                               const void* bias, void* y, int64_t M, int64_t N, int64_t K,
+                               int64_t gs, int dt, hipStream_t stream, int fmt,
+                               const LoraEp& lora);
+hipError_t launch_gemm_f32_bwd(const void* gy, const uint8_t* packed, const uint16_t* scales,
+                               void* gx, float* part, int splits, int64_t M, int64_t N, int64_t K,
+                               int64_t gs, int dt, hipStream_t stream, int fmt);
+
+// y[M, N] = the sum of `splits` fp32 partial results (split_stride(M, N) apart) + bias +
+// adapter, rounded once to dtype.
+hipError_t launch_split_reduce(const float* part, int splits, const void* bias, void* y,
+                               int64_t M, int64_t N, int dt, hipStream_t stream,
+                               const LoraEp& lora);
+
 }  // namespace ojx
 
 namespace ojx {
