@@ -17,15 +17,17 @@
 // Decoded weights follow the reference's dtype rule (coord * scales.to(dtype), rounded to
 // dtype for 2-bit and 1-bit codes); products and sums are fp32.
 //
-// Bound: the decode (about 30 VALU per code) and 8 matrix instructions of 32 cycles per 512
-// weights and 16 activation rows; the loads are small.  Rows are split over the workgroup's
-// waves (LDS reduction), the backward's also over workgroups (fp32 partial sums in the
-// caller's workspace), since one 16-row tile is a long serial chain of little work.
+// Bound: the 8 matrix instructions of 32 cycles per 512 weights and 16 activation rows (12.5 us
+// for M = 16 of 14336 x 4096) and the decode's 20-30 VALU per code, which share a SIMD's issue
+// slots, plus the first loads' round trip in short launches.  Rows are split over the
+// workgroup's waves (LDS reduction), the backward's also over workgroups (fp32 partial sums
+// in the caller's workspace), since one 16-row tile is a long serial chain of little work.
 // Measured against the 64 x 64 SIMT tiles of e8t_gemm_generic.hip (which decode every weight
-// separately, from the flat index, and leave most of the chip idle at few rows), ternary in
-// fp32: forward M = 1 of 4096 x 4096 (gs 32) 703 -> 15.9 us, M = 16 of 14336 x 4096 (gs 64)
-// 773 -> 58 us; backward dX of the latter 3917 -> 38.6 us with its reduction.  Error against
-// 64-bit sums 9e-7 -> 3e-7 (2-norm): each wave's chain is a fraction of K.
+// separately, from the flat index, and leave most of the chip idle at few rows), ternary
+// gs 32 in fp32, us from a graph: forward M = 1 of 4096 x 4096 706 -> 9, M = 16 of 14336 x 4096
+// 742 -> 30, M = 64 816 -> 83; backward dX (with its reduction) M = 1 of 4096 x 4096 849 ->
+// 14.6, M = 16 of 14336 x 4096 3940 -> 33, M = 64 4595 -> 83.  Error against 64-bit sums
+// 9e-7 -> 3e-7 (2-norm): each wave's chain is a fraction of K.
 
 #include "e8t_device.h"
 #include "e8t_internal.h"
@@ -35,10 +37,6 @@
 namespace ojx {
 
 namespace {
-
-// Values that lanes outside the matrix read as their activations.
-__device__ const float __attribute__((aligned(16))) kZeros8[8] = {0.f, 0.f, 0.f, 0.f,
-                                                                 0.f, 0.f, 0.f, 0.f};
 
 // Table of coordinate quads (float4) per format: ternary the 102 four-digit halves of raw =
 // 2 * code (81 of them valid), 2-bit the 256 code bytes, 1-bit two quads per code.
@@ -64,29 +62,17 @@ __device__ __forceinline__ void fill_quads(float4* tab) {
     }
 }
 
-// The codes of one weight row: load(t) fetches the two bytes (1-bit: one) that hold code t,
-// code() takes its bits out of them.
-template <int FMT>
-struct CodeRow {
-    const uint8_t* p;
-    uint32_t odd;  // ternary: the row starts in the middle of a 3-byte pair
-
-    CodeRow() = default;
-    __device__ __forceinline__ CodeRow(const uint8_t* packed, int64_t first) {
-        odd = FMT == kFmtTernary ? (uint32_t)(first & 1) : 0u;
-        p = packed + (FMT == kFmtTernary ? 3 * (first >> 1) : FMT == kFmt2Bit ? 2 * first : first);
-    }
-    __device__ __forceinline__ uint32_t load(uint32_t t) const {
-        if constexpr (FMT == kFmtRoot) return p[t];
-        uint16_t v;
-        __builtin_memcpy(&v, p + (FMT == kFmtTernary ? (3u * (t + odd)) >> 1 : 2u * t), 2);
-        return v;
-    }
-    // bits of code t as load() returned them
-    __device__ __forceinline__ uint32_t code(uint32_t raw, uint32_t t) const {
-        return FMT == kFmtTernary ? (raw >> (4u * ((t + odd) & 1u))) & 0xFFFu : raw;
-    }
-};
+// Code t of a row (rows start on a byte: a ternary row holds whole pairs of codes, K % 16 ==
+// 0) lies in the two bytes (1-bit: one) from code_byte(t); code_of takes its bits from them.
+template <int FMT> __device__ __forceinline__ uint32_t code_byte(uint32_t t) {
+    return FMT == kFmtTernary ? (3u * t) >> 1 : FMT == kFmt2Bit ? 2u * t : t;
+}
+template <int FMT> __device__ __forceinline__ uint32_t code_of(uint32_t raw, uint32_t t) {
+    return FMT == kFmtTernary ? (raw >> (4u * (t & 1u))) & 0xFFFu : raw;
+}
+template <int FMT> __host__ __device__ constexpr int64_t row_bytes(int64_t codes) {
+    return FMT == kFmtTernary ? 3 * codes / 2 : FMT == kFmt2Bit ? 2 * codes : codes;
+}
 
 template <int FMT, int DT>
 __device__ __forceinline__ void decode8(const float4* tab, uint32_t code, float s, float (&w)[8]) {
@@ -123,15 +109,16 @@ template <int DT, int n> struct RawX {
     static constexpr int W = DT == kF32 ? n : n / 2;
     uint32_t w[W];
 
-    __device__ __forceinline__ void load(const char* p) {
+    // byte offset vo; kNoRecordOffset (or any offset past the buffer) reads zeros
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, uint32_t vo) {
         if constexpr (W % 4 == 0) {
 #pragma unroll
             for (int i = 0; i < W / 4; ++i) {
-                const uint4 v = reinterpret_cast<const uint4*>(p)[i];
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, vo + 16u * i, 0, 0);
                 w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
             }
         } else {
-            const uint2 v = *reinterpret_cast<const uint2*>(p);
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(b, vo, 0, 0);
             w[0] = v.x; w[1] = v.y;
         }
     }
@@ -142,106 +129,26 @@ template <int DT, int n> struct RawX {
     }
 };
 
-template <int DT> constexpr int esize() { return DT == kF32 ? 4 : 2; }
+template <int DT> constexpr uint32_t esize() { return DT == kF32 ? 4 : 2; }
+
+// Buffer over `rows` rows of a row-major [M, width] matrix from row m0 (fewer at its end).
+template <int DT>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const void* a, int64_t m0, int64_t M,
+                                                              int64_t width, int rows) {
+    const int64_t left = M - m0 < rows ? M - m0 : rows;
+    return __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(static_cast<const char*>(a) + m0 * width * esize<DT>()), (short)0,
+        (int)(left * width * esize<DT>()), kRsrcWord3);
+}
 
 }  // namespace
 
-// y[M, N] = x . W^T (+ bias, + adapter).  MT: 16-row activation tiles per wave, R: 16-row
-// weight tiles per wave, NW: waves of the workgroup (they split K), U: 32-k blocks fetched
-// together, one group of them ahead of the one being contracted.
-template <int FMT, int DT, int MT, int R, int NW, int U>
-__global__ __launch_bounds__(64 * NW) void gemm_f32_fwd(
-    const void* __restrict__ x, const uint8_t* __restrict__ packed,
-    const uint16_t* __restrict__ scales, const void* __restrict__ bias, void* __restrict__ y,
-    int64_t M, int64_t N, int64_t K, int gs_shift, LoraEp lora) {
-    __shared__ float4 tab[quad_entries<FMT>()];
-    __shared__ float red[NW * MT * R * 256];
+// The waves' partial sums (acc: this wave's tiles, through `red`), then one store per output.
+template <int DT, int MT, int R, int NW>
+__device__ __forceinline__ void f32_fwd_store(const f32x4 (&acc)[MT][R], float* red,
+                                              const void* bias, void* y, int64_t M, int64_t N,
+                                              int64_t m0, int64_t n0, const LoraEp& lora) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, i16 = lane & 15;
-    const int64_t n0 = (int64_t)blockIdx.x * (16 * R), m0 = (int64_t)blockIdx.y * (16 * MT);
-    fill_quads<FMT>(tab);
-
-    const uint32_t codes = (uint32_t)(K >> 3);  // per row
-    const uint32_t blocks = (codes + 3) >> 2, per = (blocks + NW - 1) / NW;
-    const uint32_t b_begin = wave * per;
-    const uint32_t b_end = b_begin + per < blocks ? b_begin + per : blocks;
-    const int ss = gs_shift - 3;  // log2 of the codes per scale group
-
-    CodeRow<FMT> row[R];
-    const uint16_t* srow[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        int64_t n = n0 + 16 * r + i16;
-        n = n < N ? n : N - 1;  // rows past N repeat the last one, never stored
-        row[r] = CodeRow<FMT>(packed, n * codes);
-        srow[r] = scales + n * (K >> gs_shift);
-    }
-    const char* xrow[MT];
-    bool xlive[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int64_t m = m0 + 16 * t + i16;
-        xlive[t] = m < M;
-        xrow[t] = static_cast<const char*>(x) + (m < M ? m : 0) * K * esize<DT>();
-    }
-
-    struct Batch {
-        uint32_t code[U][R], sc[U][R];
-        RawX<DT, 8> xa[U][MT];
-    };
-    auto load = [&](Batch& f, uint32_t b) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t c = 4 * (b + u) + g;
-            const bool live = b + u < b_end && c < codes;
-            const uint32_t t = live ? c : 0u;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                f.code[u][r] = row[r].load(t);
-                f.sc[u][r] = srow[r][t >> ss];
-            }
-#pragma unroll
-            for (int q = 0; q < MT; ++q)
-                f.xa[u][q].load(live && xlive[q] ? xrow[q] + (int64_t)t * (8 * esize<DT>())
-                                                 : reinterpret_cast<const char*>(kZeros8));
-        }
-    };
-    f32x4 acc[MT][R];
-#pragma unroll
-    for (int q = 0; q < MT; ++q)
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[q][r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](const Batch& f, uint32_t b) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t c = 4 * (b + u) + g;
-            const bool live = b + u < b_end && c < codes;
-            const uint32_t t = live ? c : 0u;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                float w[8];
-                decode8<FMT, DT>(tab, row[r].code(f.code[u][r], t),
-                                 live ? scale_for<DT>(f.sc[u][r]) : 0.f, w);
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-#pragma unroll
-                    for (int q = 0; q < MT; ++q)
-                        acc[q][r] = mfma4(f.xa[u][q].get(j), w[j], acc[q][r]);
-            }
-        }
-    };
-
-    Batch f0, f1;
-    load(f0, b_begin);
-    __syncthreads();  // table ready
-    for (uint32_t b = b_begin; b < b_end; b += 2 * U) {
-        load(f1, b + U);
-        compute(f0, b);
-        load(f0, b + 2 * U);
-        if (b + U < b_end) compute(f1, b + U);
-    }
-
-    // the waves' partial sums, then one store per output
 #pragma unroll
     for (int q = 0; q < MT; ++q)
 #pragma unroll
@@ -263,68 +170,388 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_fwd(
     }
 }
 
+// y[M, N] = x . W^T (+ bias, + adapter).  MT: 16-row activation tiles per wave, R: 16-row
+// weight tiles per wave, NW: waves of the workgroup (they split K), U: 32-k blocks fetched
+// together, one group of them ahead of the one being contracted.  This form reads every code
+// and scale on its own, so it takes any row length.
+template <int FMT, int DT, int MT, int R, int NW, int U>
+__global__ __launch_bounds__(64 * NW) void gemm_f32_fwd(
+    const void* __restrict__ x, const uint8_t* __restrict__ packed,
+    const uint16_t* __restrict__ scales, const void* __restrict__ bias, void* __restrict__ y,
+    int64_t M, int64_t N, int64_t K, int gs_shift, LoraEp lora) {
+    __shared__ float4 tab[quad_entries<FMT>()];
+    __shared__ float red[NW * MT * R * 256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int g = lane >> 4, i16 = lane & 15;
+    const int64_t n0 = (int64_t)blockIdx.x * (16 * R), m0 = (int64_t)blockIdx.y * (16 * MT);
+    fill_quads<FMT>(tab);
+
+    const uint32_t codes = (uint32_t)(K >> 3);  // per row
+    const uint32_t blocks = (codes + 3) >> 2, per = (blocks + NW - 1) / NW;
+    const uint32_t b_begin = wave * per;
+    const uint32_t b_end = b_begin + per < blocks ? b_begin + per : blocks;
+    const int ss = gs_shift - 3;  // log2 of the codes per scale group
+
+    const uint8_t* row[R];
+    const uint16_t* srow[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        int64_t n = n0 + 16 * r + i16;
+        n = n < N ? n : N - 1;  // rows past N repeat the last one, never stored
+        row[r] = packed + n * row_bytes<FMT>(codes);
+        srow[r] = scales + n * (K >> gs_shift);
+    }
+    // activation rows m0 ..: rows past M lie past the buffer's end and read zeros
+    const __amdgpu_buffer_rsrc_t xr = rows_buffer<DT>(x, m0, M, K, 16 * MT);
+    uint32_t xrow[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xrow[t] = (uint32_t)(16 * t + i16) * (uint32_t)K * esize<DT>();
+
+    struct Batch {
+        uint32_t code[U][R], sc[U][R];
+        RawX<DT, 8> xa[U][MT];
+    };
+    auto load = [&](Batch& f, uint32_t b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t c = 4 * (b + u) + g;
+            const bool live = b + u < b_end && c < codes;
+            const uint32_t t = live ? c : 0u;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                f.code[u][r] = 0;
+                __builtin_memcpy(&f.code[u][r], row[r] + code_byte<FMT>(t),
+                                 FMT == kFmtRoot ? 1 : 2);
+                f.sc[u][r] = srow[r][t >> ss];
+            }
+#pragma unroll
+            for (int q = 0; q < MT; ++q)
+                f.xa[u][q].load(xr, live ? xrow[q] + t * (8 * esize<DT>()) : kNoRecordOffset);
+        }
+    };
+    // a wave with one tile alternates between two accumulators: back-to-back instructions
+    // then never wait for each other's result
+    constexpr int NA = MT * R == 1 ? 2 : 1;
+    f32x4 acc[NA][MT][R];
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int q = 0; q < MT; ++q)
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[a][q][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const Batch& f, uint32_t b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t c = 4 * (b + u) + g;
+            const bool live = b + u < b_end && c < codes;
+            const uint32_t t = live ? c : 0u;
+            float w[R][8];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                decode8<FMT, DT>(tab, code_of<FMT>(f.code[u][r], t),
+                                 live ? scale_for<DT>(f.sc[u][r]) : 0.f, w[r]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int q = 0; q < MT; ++q)
+                        acc[j % NA][q][r] =
+                            mfma4(f.xa[u][q].get(j), w[r][j], acc[j % NA][q][r]);
+        }
+    };
+
+    // the loads of a batch all go out before the previous batch is contracted (left to
+    // itself the scheduler sinks them towards their uses)
+    Batch f0, f1;
+    load(f0, b_begin);
+    __syncthreads();  // table ready
+    for (uint32_t b = b_begin; b < b_end; b += 2 * U) {
+        load(f1, b + U);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(f0, b);
+        load(f0, b + 2 * U);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b + U < b_end) compute(f1, b + U);
+    }
+    if constexpr (NA == 2) acc[0][0][0] += acc[NA - 1][0][0];
+
+    f32_fwd_store<DT, MT, R, NW>(acc[0], red, bias, y, M, N, m0, n0, lora);
+}
+
+// The same product where rows hold whole 4-byte words of codes and scales (f32_wide_ok): a
+// lane loads the eight consecutive codes 8 g .. 8 g + 7 of its row's 256-k chunk, and their
+// scales, in one load each, and a 4 x 4 transpose over the lane groups hands it the codes
+// 4 u + g, u = 0..7, that its activations belong to (activations are best read four lanes to a
+// 128-byte line).  Codes and scales run one chunk ahead, activations XU blocks ahead.
+// The two-byte loads and their addresses bound the form above: M = 1 / 16 of 14336 x 4096
+// (ternary, gs 32) 45 / 56 us there and 25 / 30 here, M = 512 of 4096 x 4096 195 and 160.
+// The transpose: register q of lane group g holds entries (q, q + 4 in the high half) of the
+// group's eight; afterwards register q holds entry 4 (2 q + h) + g, h the half.
+__device__ __forceinline__ void transpose_groups(uint32_t (&q)[4]) {
+    auto s = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false);
+    q[0] = s[0]; q[2] = s[1];
+    s = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
+    q[1] = s[0]; q[3] = s[1];
+    s = __builtin_amdgcn_permlane16_swap(q[0], q[1], false, false);
+    q[0] = s[0]; q[1] = s[1];
+    s = __builtin_amdgcn_permlane16_swap(q[2], q[3], false, false);
+    q[2] = s[0]; q[3] = s[1];
+}
+
+// A lane's eight codes as loaded, and as 16-bit pairs (t, t + 4).
+template <int FMT> struct WideRow {
+    static constexpr int W = FMT == kFmtTernary ? 3 : FMT == kFmt2Bit ? 4 : 2;
+    static constexpr uint32_t kBytes = 4 * W;  // of eight codes
+    uint32_t d[W];
+
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, uint32_t vo) {
+        if constexpr (W == 3) {
+            const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(b, vo, 0, 0);
+            d[0] = v.x; d[1] = v.y; d[2] = v.z;
+        } else if constexpr (W == 4) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, vo, 0, 0);
+            d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+        } else {
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(b, vo, 0, 0);
+            d[0] = v.x; d[1] = v.y;
+        }
+    }
+    __device__ __forceinline__ void pairs(uint32_t (&q)[4]) const {
+        if constexpr (FMT == kFmtTernary) {
+            const uint32_t c2 = __builtin_amdgcn_alignbit(d[1], d[0], 24) & 0xFFFu;
+            const uint32_t c5 = __builtin_amdgcn_alignbit(d[2], d[1], 28) & 0xFFFu;
+            q[0] = (d[0] & 0xFFFu) | (d[1] & 0x0FFF0000u);
+            q[1] = ((d[0] >> 12) & 0xFFFu) | (c5 << 16);
+            q[2] = c2 | ((d[2] << 8) & 0x0FFF0000u);
+            q[3] = ((d[1] >> 4) & 0xFFFu) | ((d[2] >> 4) & 0x0FFF0000u);
+        } else if constexpr (FMT == kFmt2Bit) {
+            q[0] = __builtin_amdgcn_perm(d[2], d[0], 0x05040100u);
+            q[1] = __builtin_amdgcn_perm(d[2], d[0], 0x07060302u);
+            q[2] = __builtin_amdgcn_perm(d[3], d[1], 0x05040100u);
+            q[3] = __builtin_amdgcn_perm(d[3], d[1], 0x07060302u);
+        } else {
+            q[0] = __builtin_amdgcn_perm(d[1], d[0], 0x0C040C00u);
+            q[1] = __builtin_amdgcn_perm(d[1], d[0], 0x0C050C01u);
+            q[2] = __builtin_amdgcn_perm(d[1], d[0], 0x0C060C02u);
+            q[3] = __builtin_amdgcn_perm(d[1], d[0], 0x0C070C03u);
+        }
+    }
+};
+
+// The scales of a lane's eight codes, GS weights to a scale (64: 64 or more, one scale).
+template <int GS> struct WideScale {
+    static constexpr int W = GS >= 32 ? 1 : 32 / GS;  // words: 1, 2 (gs 16), 4 (gs 8)
+    uint32_t d[W];
+
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, uint32_t vo) {
+        if constexpr (GS >= 64) {
+            d[0] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(b, vo, 0, 0);
+        } else if constexpr (W == 1) {
+            d[0] = __builtin_amdgcn_raw_buffer_load_b32(b, vo, 0, 0);
+        } else if constexpr (W == 2) {
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(b, vo, 0, 0);
+            d[0] = v.x; d[1] = v.y;
+        } else {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, vo, 0, 0);
+            d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+        }
+    }
+    __device__ __forceinline__ void pairs(uint32_t (&q)[4]) const {
+        if constexpr (GS >= 64) {
+            q[0] = q[1] = q[2] = q[3] = d[0] * 0x10001u;
+        } else if constexpr (GS == 32) {  // the scales of codes 0..3 and 4..7
+            q[0] = q[1] = q[2] = q[3] = d[0];
+        } else if constexpr (GS == 16) {
+            q[0] = q[1] = __builtin_amdgcn_perm(d[1], d[0], 0x05040100u);
+            q[2] = q[3] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
+        } else {
+            q[0] = __builtin_amdgcn_perm(d[2], d[0], 0x05040100u);
+            q[1] = __builtin_amdgcn_perm(d[2], d[0], 0x07060302u);
+            q[2] = __builtin_amdgcn_perm(d[3], d[1], 0x05040100u);
+            q[3] = __builtin_amdgcn_perm(d[3], d[1], 0x07060302u);
+        }
+    }
+};
+
+template <int FMT, int DT, int GS, int MT, int R, int NW, int XU>
+__global__ __launch_bounds__(64 * NW) void gemm_f32_fwd_wide(
+    const void* __restrict__ x, const uint8_t* __restrict__ packed,
+    const uint16_t* __restrict__ scales, const void* __restrict__ bias, void* __restrict__ y,
+    int64_t M, int64_t N, int64_t K, int gs_shift, LoraEp lora) {
+    using Row = WideRow<FMT>;
+    __shared__ float4 tab[quad_entries<FMT>()];
+    __shared__ float red[NW * MT * R * 256];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, i16 = lane & 15;
+    const int64_t n0 = (int64_t)blockIdx.x * (16 * R), m0 = (int64_t)blockIdx.y * (16 * MT);
+
+    const int codes = (int)(K >> 3);  // per row
+    const int chunks = (codes + 31) >> 5, per = (chunks + NW - 1) / NW;
+    const int c_begin = wave * per;
+    const int c_end = c_begin + per < chunks ? c_begin + per : chunks;
+
+    // the workgroup's rows of codes and scales; rows past N lie past the end and read zeros
+    const int64_t left = N - n0 < 16 * R ? N - n0 : 16 * R;
+    const uint32_t rowbytes = (uint32_t)row_bytes<FMT>(codes);
+    const uint32_t srowbytes = (uint32_t)(K >> gs_shift) * 2;
+    const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(packed + n0 * rowbytes), (short)0, (int)(left * rowbytes), kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(reinterpret_cast<const char*>(scales) + n0 * srowbytes), (short)0,
+        (int)(left * srowbytes), kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t xr = rows_buffer<DT>(x, m0, M, K, 16 * MT);
+
+    Row cd[R];
+    WideScale<GS> sc[R];
+    auto load_w = [&](int ch) {  // a chunk past the last reads zeros or a later row, unused
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t row = 16 * r + i16, c = 32 * ch + 8 * g;
+            cd[r].load(pr, row * rowbytes + (c >> 3) * Row::kBytes);
+            sc[r].load(sr, row * srowbytes + ((c << 3) >> gs_shift) * 2);
+        }
+    };
+    struct XBatch { RawX<DT, 8> a[XU][MT]; };
+    auto load_x = [&](XBatch& f, int ch, int u0) {
+#pragma unroll
+        for (int u = 0; u < XU; ++u) {
+            const int c = 32 * ch + 4 * (u0 + u) + g;
+            const bool live = c < codes && ch < c_end;
+#pragma unroll
+            for (int q = 0; q < MT; ++q)
+                f.a[u][q].load(xr, live ? (uint32_t)((16 * q + i16) * codes + c) * (8 * esize<DT>())
+                                        : kNoRecordOffset);
+        }
+    };
+    // one tile per wave: two accumulators, so that instructions in a row never wait for each
+    // other's result
+    constexpr int NA = MT * R == 1 ? 2 : 1;
+    f32x4 acc[NA][MT][R];
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int q = 0; q < MT; ++q)
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[a][q][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    XBatch xb[2];
+    load_w(c_begin);
+    load_x(xb[0], c_begin, 0);
+    fill_quads<FMT>(tab);
+    __syncthreads();  // table ready
+    for (int ch = c_begin; ch < c_end; ++ch) {
+        uint32_t cq[R][4], sq[R][4];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            cd[r].pairs(cq[r]);
+            sc[r].pairs(sq[r]);
+            transpose_groups(cq[r]);
+            transpose_groups(sq[r]);
+        }
+        load_w(ch + 1);
+#pragma unroll
+        for (int u0 = 0; u0 < 8; u0 += XU) {
+            const XBatch& xc = xb[(u0 / XU) & 1];
+            load_x(xb[(u0 / XU + 1) & 1], u0 + XU < 8 ? ch : ch + 1, (u0 + XU) & 7);
+            __builtin_amdgcn_sched_barrier(0);  // the loads go out before the contraction
+#pragma unroll
+            for (int u = 0; u < XU; ++u) {
+                const int e = u0 + u;
+                const bool live = 32 * ch + 4 * e + g < codes;
+                float w[R][8];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const uint32_t code = e & 1 ? cq[r][e >> 1] >> 16 : cq[r][e >> 1] & 0xFFFFu;
+                    const uint32_t s16 = e & 1 ? sq[r][e >> 1] >> 16 : sq[r][e >> 1] & 0xFFFFu;
+                    decode8<FMT, DT>(tab, code, live ? scale_for<DT>(s16) : 0.f, w[r]);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+#pragma unroll
+                        for (int q = 0; q < MT; ++q)
+                            acc[j % NA][q][r] =
+                                mfma4(xc.a[u][q].get(j), w[r][j], acc[j % NA][q][r]);
+            }
+        }
+    }
+    if constexpr (NA == 2) acc[0][0][0] += acc[NA - 1][0][0];
+    f32_fwd_store<DT, MT, R, NW>(acc[0], red, bias, y, M, N, m0, n0, lora);
+}
+
 // gx[M, K] = gy . W, or (gridDim.z > 1) the fp32 partial sums of row range blockIdx.z in
 // part[z][M][K].  VEC: N % 4 == 0 and gy aligned for loads of four values.
 template <int FMT, int DT, int MT, int NW, bool VEC>
-__global__ __launch_bounds__(64 * NW) void gemm_f32_bwd(
+__global__ __launch_bounds__(64 * NW, 2) void gemm_f32_bwd(
     const void* __restrict__ gy, const uint8_t* __restrict__ packed,
     const uint16_t* __restrict__ scales, void* __restrict__ gx, float* __restrict__ part,
     int64_t M, int64_t N, int64_t K, int gs_shift) {
     __shared__ float4 tab[quad_entries<FMT>()];
     __shared__ f32x4 red[NW / 2][MT * 8][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, i16 = lane & 15;
     const int64_t m0 = (int64_t)blockIdx.y * (16 * MT);
-    fill_quads<FMT>(tab);
 
     const uint32_t codes = (uint32_t)(K >> 3);
     const uint32_t c = 16 * blockIdx.x + i16;
     const uint32_t cc = c < codes ? c : codes - 1;  // columns past K are never stored
-    const uint32_t sidx = cc >> (gs_shift - 3);
-    const int64_t sld = K >> gs_shift;
-    const int64_t groups = (N + 15) >> 4;  // 16 rows: four instructions' worth per lane group
-    const int64_t parts = (int64_t)gridDim.z * NW, p = (int64_t)blockIdx.z * NW + wave;
-    const int64_t q_begin = groups * p / parts, q_end = groups * (p + 1) / parts;
+    const int groups = (int)((N + 15) >> 4);  // 16 rows: four instructions per lane group
+    const int parts = gridDim.z * NW, p = blockIdx.z * NW + wave;
+    const int q_begin = (int)((int64_t)groups * p / parts);
+    const int q_end = (int)((int64_t)groups * (p + 1) / parts);
 
-    const char* yrow[MT];
-    bool ylive[MT];
+    // rows past N lie past the buffers' ends: zero codes, zero scales
+    const uint32_t rowbytes = (uint32_t)row_bytes<FMT>(codes);
+    const uint32_t srowbytes = (uint32_t)(K >> gs_shift) * 2;
+    const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)packed, (short)0, (int)(N * rowbytes), kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)scales, (short)0, (int)(N * srowbytes), kRsrcWord3);
+    uint32_t vo_code[4], vo_scale[4];  // of row 4 g + s of a group, column code c
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int64_t m = m0 + 16 * t + i16;
-        ylive[t] = m < M;
-        yrow[t] = static_cast<const char*>(gy) + (m < M ? m : 0) * N * esize<DT>();
+    for (int s = 0; s < 4; ++s) {
+        vo_code[s] = (4 * g + s) * rowbytes + code_byte<FMT>(cc);
+        vo_scale[s] = (4 * g + s) * srowbytes + (cc >> (gs_shift - 3)) * 2;
     }
+
+    const __amdgpu_buffer_rsrc_t yr = rows_buffer<DT>(gy, m0, M, N, 16 * MT);
+    uint32_t yrow[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) yrow[t] = (uint32_t)(16 * t + i16) * (uint32_t)N * esize<DT>();
     struct Batch {
-        uint32_t code[4], sc[4], odd;
+        uint32_t code[4], sc[4];
         RawX<DT, 4> ya[MT];
     };
     // rows n = 16 q + 4 g + s, s = 0..3
-    auto load = [&](Batch& f, int64_t q) {
+    auto load = [&](Batch& f, int q) {
         q = q < q_end ? q : q_end - 1;  // a group past the last is loaded again, never used
-        const int64_t n0 = 16 * q + 4 * g;
-        f.odd = 0;
+        const int64_t n0 = 16 * (int64_t)q + 4 * g;
+        const int so = uniform_offset(16 * (int64_t)q * rowbytes);
+        const int ss = uniform_offset(16 * (int64_t)q * srowbytes);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const int64_t n = n0 + s < N ? n0 + s : N - 1;
-            const CodeRow<FMT> row(packed, n * codes);
-            f.code[s] = row.load(cc);
-            f.odd |= row.odd << s;
-            f.sc[s] = scales[n * sld + sidx];
+            if constexpr (FMT == kFmtRoot)
+                f.code[s] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(pr, vo_code[s], so, 0);
+            else
+                f.code[s] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(pr, vo_code[s], so, 0);
+            f.sc[s] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sr, vo_scale[s], ss, 0);
         }
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             if constexpr (VEC) {
-                f.ya[t].load(ylive[t] && n0 < N ? yrow[t] + n0 * esize<DT>()
-                                                : reinterpret_cast<const char*>(kZeros8));
+                f.ya[t].load(yr, n0 < N ? yrow[t] + (uint32_t)n0 * esize<DT>() : kNoRecordOffset);
             } else {
                 uint32_t v[4];
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const char* a = ylive[t] && n0 + s < N
-                                        ? yrow[t] + (n0 + s) * esize<DT>()
-                                        : reinterpret_cast<const char*>(kZeros8);
-                    if constexpr (DT == kF32) v[s] = *reinterpret_cast<const uint32_t*>(a);
-                    else v[s] = *reinterpret_cast<const uint16_t*>(a);
+                    const uint32_t vo =
+                        n0 + s < N ? yrow[t] + (uint32_t)(n0 + s) * esize<DT>() : kNoRecordOffset;
+                    if constexpr (DT == kF32) v[s] = __builtin_amdgcn_raw_buffer_load_b32(yr, vo, 0, 0);
+                    else v[s] = __builtin_amdgcn_raw_buffer_load_b16(yr, vo, 0, 0);
                 }
                 if constexpr (DT == kF32) {
 #pragma unroll
@@ -341,15 +568,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_bwd(
     for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](const Batch& f, int64_t q) {
-        const int64_t n0 = 16 * q + 4 * g;
+    auto compute = [&](const Batch& f) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            uint32_t code = f.code[s];
-            if constexpr (FMT == kFmtTernary)
-                code = (code >> (4u * ((cc + ((f.odd >> s) & 1u)) & 1u))) & 0xFFFu;
             float w[8];
-            decode8<FMT, DT>(tab, code, n0 + s < N ? scale_for<DT>(f.sc[s]) : 0.f, w);
+            decode8<FMT, DT>(tab, code_of<FMT>(f.code[s], cc), scale_for<DT>(f.sc[s]), w);
 #pragma unroll
             for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -359,12 +582,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_bwd(
 
     Batch f0, f1;
     if (q_begin < q_end) load(f0, q_begin);
+    fill_quads<FMT>(tab);
     __syncthreads();  // table ready
-    for (int64_t q = q_begin; q < q_end; q += 2) {
+    for (int q = q_begin; q < q_end; q += 2) {
         load(f1, q + 1);
-        compute(f0, q);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(f0);
         load(f0, q + 2);
-        if (q + 1 < q_end) compute(f1, q + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (q + 1 < q_end) compute(f1);
     }
 
     // the waves' sums, halving: waves [h, 2h) hand theirs to waves [0, h)
@@ -410,19 +636,24 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_bwd(
 bool gemm_f32_supported(const void* x, const uint8_t* packed, const uint16_t* scales, int64_t M,
                         int64_t N, int64_t K, int64_t gs, int fmt, bool bwd) {
     // rows hold whole codes and whole scale groups of 2^t >= 8 weights (a ternary group is a
-    // multiple of 16); the kernels index a row's codes and the grid in 32 bits
+    // multiple of 16); 64 activation rows stay below 2^31 bytes (32-bit buffer offsets)
     if (gs < 8 || (gs & (gs - 1)) != 0 || gs > (1ll << 30) || K < gs || K % gs != 0) return false;
-    if (M < 1 || N < 1 || K >= (1ll << 31) || N >= (1ll << 31) || (M + 15) / 16 > 65535)
+    if (M < 1 || N < 1 || K >= (1ll << 23) || N >= (bwd ? 1ll << 23 : 1ll << 31) ||
+        (M + 15) / 16 > 65535)
         return false;
     // 16-byte loads of eight activations along K (the backward picks its loads by N)
     if (!bwd && ((uintptr_t)x & 15u)) return false;
+    // the backward addresses whole weight buffers in 32 bits, a group of rows past the end
+    if (bwd && (N + 16) * (K / 4) >= (1ll << 31)) return false;
+    if (bwd && (N + 16) * (K / gs * 2) >= (1ll << 31)) return false;
     if (bwd && ((uintptr_t)x & 3u)) return false;
     return ((uintptr_t)scales & 1u) == 0;
 }
 
-// Row splits of the backward over workgroups: towards kF32Waves waves on the chip (two per
-// SIMD), while every wave keeps at least four groups of 16 rows.
-constexpr int64_t kF32Waves = 2048;
+// Row splits of the backward over workgroups: towards kF32Waves waves on the chip (four per
+// SIMD; with two, M = 1 and 16 of 14336 x 4096 took 33.3 and 34.9 us against 30.1 and 32.7),
+// while every wave keeps at least four groups of 16 rows.
+constexpr int64_t kF32Waves = 4096;
 constexpr int kF32BwdWaves = 8;
 
 static int f32_row_tiles(int64_t M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
@@ -438,14 +669,36 @@ int gemm_f32_bwd_splits(int64_t M, int64_t N, int64_t K) {
     return s < 1 ? 1 : (int)s;
 }
 
-template <int FMT, int DT, int MT, int R, int NW, int U>
+// Rows of whole 4-byte words: codes 12 (ternary), 16 (2-bit) or 8 (1-bit) bytes per 64
+// weights, and scales of two bytes (groups of 64 and more are read one scale at a time).
+static bool f32_wide_ok(const uint8_t* packed, const uint16_t* scales, int64_t K, int64_t gs,
+                        int fmt) {
+    const int64_t row16 = K / 16 * (fmt == kFmtTernary ? 3 : fmt == kFmt2Bit ? 4 : 2);
+    return K % 16 == 0 && row16 % 4 == 0 && (gs >= 64 || (K / gs) % 2 == 0) &&
+           (((uintptr_t)packed | (uintptr_t)scales) & 3u) == 0;
+}
+
+template <int FMT, int DT, int MT, int R, int NW>
 static hipError_t launch_f32_fwd_cfg(const void* x, const uint8_t* packed, const uint16_t* scales,
                                      const void* bias, void* y, int64_t M, int64_t N, int64_t K,
-                                     int gs_shift, hipStream_t s, const LoraEp& lora) {
+                                     int sh, hipStream_t s, const LoraEp& lora) {
+    constexpr int XU = MT == 4 ? 1 : 2;
     const dim3 grid((unsigned)((N + 16 * R - 1) / (16 * R)),
                     (unsigned)((M + 16 * MT - 1) / (16 * MT)));
-    hipLaunchKernelGGL((gemm_f32_fwd<FMT, DT, MT, R, NW, U>), grid, dim3(64 * NW), 0, s, x, packed,
-                       scales, bias, y, M, N, K, gs_shift, lora);
+#define OJX_LAUNCH(...)                                                                          \
+    hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(64 * NW), 0, s, x, packed, scales, bias, y, M,  \
+                       N, K, sh, lora)
+    if (!f32_wide_ok(packed, scales, K, (int64_t)1 << sh, FMT))
+        OJX_LAUNCH(gemm_f32_fwd<FMT, DT, MT, R, NW, XU>);
+    else if (sh >= 6)
+        OJX_LAUNCH(gemm_f32_fwd_wide<FMT, DT, 64, MT, R, NW, XU>);
+    else if (sh == 5)
+        OJX_LAUNCH(gemm_f32_fwd_wide<FMT, DT, 32, MT, R, NW, XU>);
+    else if (sh == 4)
+        OJX_LAUNCH(gemm_f32_fwd_wide<FMT, DT, 16, MT, R, NW, XU>);
+    else if constexpr (FMT != kFmtTernary)  // ternary groups are multiples of 16
+        OJX_LAUNCH(gemm_f32_fwd_wide<FMT, DT, 8, MT, R, NW, XU>);
+#undef OJX_LAUNCH
     return hipGetLastError();
 }
 
@@ -453,23 +706,20 @@ template <int FMT, int DT>
 static hipError_t launch_f32_fwd_t(const void* x, const uint8_t* packed, const uint16_t* scales,
                                    const void* bias, void* y, int64_t M, int64_t N, int64_t K,
                                    int sh, hipStream_t s, const LoraEp& lora) {
+    // Weight tiles per wave: one while that leaves at most two workgroups per CU, then two,
+    // which share the activations' loads (M = 16, ternary gs 32: 4096 x 4096 12.5 against
+    // 16.3 us, 14336 x 4096 39.8 against 29.7; four tiles 28.4 and 29.7).  Eight waves share
+    // a row's K (4 and 16 waves: 10.4 and 9.1 against 9.1 us at M = 1 of 4096 x 4096); at
+    // M > 32 a wave's matrix work is long enough for four (M = 512 148.8 against 155.7 us).
     const int mt = f32_row_tiles(M);
-    const int64_t tiles = (N + 15) / 16;
-    if (mt == 1) {
-        if (tiles >= 512)
-            return launch_f32_fwd_cfg<FMT, DT, 1, 2, 8, 4>(x, packed, scales, bias, y, M, N, K, sh,
-                                                           s, lora);
-        return launch_f32_fwd_cfg<FMT, DT, 1, 1, 8, 4>(x, packed, scales, bias, y, M, N, K, sh, s,
-                                                       lora);
-    }
-    if (mt == 2)
-        return launch_f32_fwd_cfg<FMT, DT, 2, 2, 8, 2>(x, packed, scales, bias, y, M, N, K, sh, s,
-                                                       lora);
-    if (tiles * ((M + 63) / 64) >= 1024)
-        return launch_f32_fwd_cfg<FMT, DT, 4, 4, 4, 1>(x, packed, scales, bias, y, M, N, K, sh, s,
-                                                       lora);
-    return launch_f32_fwd_cfg<FMT, DT, 4, 2, 8, 1>(x, packed, scales, bias, y, M, N, K, sh, s,
-                                                   lora);
+    const int64_t wgs = (N + 15) / 16 * ((M + 16 * mt - 1) / (16 * mt));
+    auto cfg = mt == 1   ? (wgs >= 512 ? launch_f32_fwd_cfg<FMT, DT, 1, 2, 8>
+                                       : launch_f32_fwd_cfg<FMT, DT, 1, 1, 8>)
+               : mt == 2 ? (wgs >= 512 ? launch_f32_fwd_cfg<FMT, DT, 2, 2, 8>
+                                       : launch_f32_fwd_cfg<FMT, DT, 2, 1, 8>)
+                         : (wgs >= 512 ? launch_f32_fwd_cfg<FMT, DT, 4, 2, 4>
+                                       : launch_f32_fwd_cfg<FMT, DT, 4, 1, 8>);
+    return cfg(x, packed, scales, bias, y, M, N, K, sh, s, lora);
 }
 
 template <int FMT, int DT, int MT, int NW>

@@ -67,6 +67,17 @@ SHAPES = [
     ("1bit", 66, 31, 104, 8, f16, True),
     ("ternary", 6, 1536, 4448, 32, f16, True),
     ("ternary", 300, 200, 96, 32, bf16, False),
+    # rows of whole words (one load per eight codes), the last 256-k chunk cut off
+    ("ternary", 4, 200, 704, 16, f32, True),
+    ("ternary", 20, 8210, 320, 64, f32, False),
+    ("ternary", 50, 5000, 576, 32, f32, True),
+    ("2bit", 16, 100, 1008, 8, f32, True),
+    ("2bit", 70, 530, 544, 16, f32, False),
+    ("2bit", 2, 72, 2304, 256, f32, False),
+    ("2bit", 3, 50, 1000, 8, bf16, False),
+    ("1bit", 2, 40, 288, 16, f32, True),
+    ("1bit", 40, 70, 1056, 8, f32, False),
+    ("1bit", 1, 100, 4128, 32, f16, True),
 ]
 
 
