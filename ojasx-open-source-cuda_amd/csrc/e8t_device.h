@@ -76,13 +76,16 @@ template <int DT> __device__ __forceinline__ float scale_for(uint32_t s16) {
 // Low-rank term of a fused forward with a LoRA adapter (E8LatticeLinear.forward,
 // lattice.py:839-842: out + scaling * ((x @ A) @ B)): y[m, n] += sum_j u[m, j] * B[j, n], with
 // u = scaling * (x @ A) in fp32 [M, r] (row stride ldu) and B the up-projection [r, N] in the
-// activation dtype (row stride ldb).  r == 0: no adapter.
+// activation dtype (row stride ldb).  r == 0: no adapter.  The backward's term has the same
+// form with gx, scaling * (gy @ B^T) and A^T in the places of y, u and B: ldn is the stride
+// between B's columns.
 struct LoraEp {
     const float* u;
     const void* b;
     int64_t r;
     int64_t ldu;
     int64_t ldb;
+    int64_t ldn = 1;
 };
 
 template <int DT>
@@ -96,7 +99,43 @@ __device__ __forceinline__ float lora_term(const float* u, const void* b, int64_
 
 template <int DT>
 __device__ __forceinline__ float lora_term(const LoraEp& l, int64_t m, int64_t n) {
-    return l.r > 0 ? lora_term<DT>(l.u, l.b, l.r, l.ldu, l.ldb, m, n) : 0.f;
+    return l.r > 0 ? lora_term<DT>(l.u, static_cast<const char*>(l.b) + n * (l.ldn - 1) *
+                                   (int64_t)sizeof(typename Elem<DT>::T), l.r, l.ldu, l.ldb, m, n)
+                   : 0.f;
+}
+
+// The same term added to 16 x 16 MFMA result tiles: acc[i][j] holds rows row0 + 16 i + 4 g + q
+// and column col(j) of this lane (g = lane / 16, its i16 = lane % 16 already in col).  Four
+// ranks per fp32 matrix instruction, so u and B enter in full precision as in lora_term;
+// per output lora_term's loads cost far more than its sums (a rank-8 adapter on 2048 x 4096
+// outputs: 49 us in the split reduction against 13 without it).  A K split shares the ranks
+// out: split `part` of `parts` adds every parts-th four of them.
+template <int DT, int TM, int TN, typename Col>
+__device__ __forceinline__ void lora_add(
+    __attribute__((ext_vector_type(4))) float (&acc)[TM][TN], const LoraEp& l, int64_t row0,
+    int64_t M, int64_t cols, int lane, Col col, int part = 0, int parts = 1) {
+    const int g = lane >> 4, i16 = lane & 15;
+#pragma unroll 2
+    for (int64_t t = 4 * part; t < l.r; t += 4 * parts) {
+        const int64_t k = t + g;
+        const bool live = k < l.r;
+        float a[TM], b[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int64_t row = row0 + 16 * i + i16;
+            a[i] = live && row < M ? l.u[row * l.ldu + k] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int64_t c = col(j);
+            b[j] = live && c < cols ? load_as_f32<DT>(l.b, k * l.ldb + c * l.ldn) : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
 }
 
 // ---------------------------------------------------------------- packed codes

@@ -145,10 +145,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const void* a, int
 
 // The waves' partial sums (acc: this wave's tiles, through `red`), then one store per output.
 template <int DT, int MT, int R, int NW>
-__device__ __forceinline__ void f32_fwd_store(const f32x4 (&acc)[MT][R], float* red,
+__device__ __forceinline__ void f32_fwd_store(f32x4 (&acc)[MT][R], float* red,
                                               const void* bias, void* y, int64_t M, int64_t N,
                                               int64_t m0, int64_t n0, const LoraEp& lora) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lora.r > 0 && wave == 0)
+        lora_add<DT, MT, R>(acc, lora, m0, M, N, lane,
+                            [&](int r) { return n0 + 16 * r + (lane & 15); });
 #pragma unroll
     for (int q = 0; q < MT; ++q)
 #pragma unroll
@@ -165,7 +168,7 @@ __device__ __forceinline__ void f32_fwd_store(const f32x4 (&acc)[MT][R], float* 
         const int64_t m = m0 + 16 * q + 4 * (l >> 4) + e, n = n0 + 16 * r + (l & 15);
         if (m < M && n < N) {
             if (bias) v += load_as_f32<DT>(bias, n);
-            store_from_f32<DT>(y, m * N + n, v + lora_term<DT>(lora, m, n));
+            store_from_f32<DT>(y, m * N + n, v);
         }
     }
 }
@@ -736,7 +739,7 @@ static hipError_t launch_f32_bwd_cfg(const void* gy, const uint8_t* packed,
                            packed, scales, gx, part, M, N, K, sh);
     const hipError_t e = hipGetLastError();
     if (splits == 1 || e != hipSuccess) return e;
-    return launch_split_reduce(part, splits, nullptr, gx, M, K, DT, s, LoraEp{});
+    return launch_split_reduce(part, splits, nullptr, gx, M, K, DT, s);
 }
 
 template <int FMT, int DT>

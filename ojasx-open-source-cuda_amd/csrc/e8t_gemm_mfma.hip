@@ -936,6 +936,9 @@ __global__ __launch_bounds__(C::THREADS) void gemm_mfma_kernel(
     }
 
     // ---- epilogue: lane (g, i16) holds rows 4g+q of column i16 of each 16x16 tile
+    if (lora.r > 0)
+        lora_add<DT, kTM, kTN>(acc, lora, m0 + arow0, M, NO, lane,
+                               [&](int j) { return n0 + brow0 + 16 * j + i16; }, split, splits);
     if (splits > 1) {  // fp32 partial sums of this K range: part[split][row][col]
         float* pp = part + (int64_t)split * split_stride(M, NO);
 #pragma unroll
@@ -964,9 +967,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_mfma_kernel(
             for (int q = 0; q < 4; ++q) {
                 const int64_t row = m0 + arow0 + 16 * i + 4 * g + q;
                 if (row < M) {
-                    float v = acc[i][j][q] + bv;
-                    if (!BWD) v += lora_term<DT>(lora, row, col);
-                    store_from_f32<DT>(y, row * NO + col, v);
+                    store_from_f32<DT>(y, row * NO + col, acc[i][j][q] + bv);
                 }
             }
         }
@@ -977,7 +978,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_mfma_kernel(
 template <int DT>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
     const float* __restrict__ part, int splits, const void* __restrict__ bias,
-    void* __restrict__ y, int64_t M, int64_t N, LoraEp lora) {
+    void* __restrict__ y, int64_t M, int64_t N) {
     const int64_t MN = M * N, stride = split_stride(M, N);
     const int64_t i4 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i4 >= MN) return;
@@ -992,31 +993,30 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
         for (int e = 0; e < 4; ++e) {
             const int64_t i = i4 + e;
             const float bv = bias ? load_as_f32<DT>(bias, i % N) : 0.f;
-            store_from_f32<DT>(y, i, v[e] + bv + lora_term<DT>(lora, i / N, i % N));
+            store_from_f32<DT>(y, i, v[e] + bv);
         }
     } else {
         for (int64_t i = i4; i < MN; ++i) {
             float a = 0.f;
             for (int s = 0; s < splits; ++s) a += part[(int64_t)s * stride + i];
             const float bv = bias ? load_as_f32<DT>(bias, i % N) : 0.f;
-            store_from_f32<DT>(y, i, a + bv + lora_term<DT>(lora, i / N, i % N));
+            store_from_f32<DT>(y, i, a + bv);
         }
     }
 }
 
 hipError_t launch_split_reduce(const float* part, int splits, const void* bias, void* y,
-                               int64_t M, int64_t N, int dt, hipStream_t stream,
-                               const LoraEp& lora) {
+                               int64_t M, int64_t N, int dt, hipStream_t stream) {
     const dim3 grid((unsigned)((M * N + 1023) / 1024));
     if (dt == kF32)
         hipLaunchKernelGGL((gemm_split_reduce_kernel<kF32>), grid, dim3(256), 0, stream, part,
-                           splits, bias, y, M, N, lora);
+                           splits, bias, y, M, N);
     else if (dt == kF16)
         hipLaunchKernelGGL((gemm_split_reduce_kernel<kF16>), grid, dim3(256), 0, stream, part,
-                           splits, bias, y, M, N, lora);
+                           splits, bias, y, M, N);
     else
         hipLaunchKernelGGL((gemm_split_reduce_kernel<kBF16>), grid, dim3(256), 0, stream, part,
-                           splits, bias, y, M, N, lora);
+                           splits, bias, y, M, N);
     return hipGetLastError();
 }
 
@@ -1058,8 +1058,7 @@ static hipError_t launch_cfg(const void* x, const uint8_t* packed, const uint16_
                        N, K, lora);
     const hipError_t e = hipGetLastError();
     if (splits == 1 || e != hipSuccess) return e;
-    return launch_split_reduce(part, splits, BWD ? nullptr : bias, y, M, NO, DT, stream,
-                               BWD ? LoraEp{} : lora);
+    return launch_split_reduce(part, splits, BWD ? nullptr : bias, y, M, NO, DT, stream);
 }
 
 // Tile configuration and K split of a launch.

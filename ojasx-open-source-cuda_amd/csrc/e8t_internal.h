@@ -83,11 +83,10 @@ hipError_t launch_gemm_f32_bwd(const void* gy, const uint8_t* packed, const uint
                                void* gx, float* part, int splits, int64_t M, int64_t N, int64_t K,
                                int64_t gs, int dt, hipStream_t stream, int fmt);
 
-// y[M, N] = the sum of `splits` fp32 partial results (split_stride(M, N) apart) + bias +
-// adapter, rounded once to dtype.
+// y[M, N] = the sum of `splits` fp32 partial results (split_stride(M, N) apart) + bias,
+// rounded once to dtype.
 hipError_t launch_split_reduce(const float* part, int splits, const void* bias, void* y,
-                               int64_t M, int64_t N, int dt, hipStream_t stream,
-                               const LoraEp& lora);
+                               int64_t M, int64_t N, int dt, hipStream_t stream);
 
 }  // namespace ojx
 
