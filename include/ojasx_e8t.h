@@ -157,6 +157,21 @@ int ojx_e8t_gemm_bwd_dx(const void* grad_y, const uint8_t* packed, const uint16_
                         void* grad_x, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype,
                         void* workspace, size_t workspace_bytes, void* stream);
 
+/* Backward of a linear with a LoRA adapter (the gradients of E8LatticeLinear.forward,
+ * lattice.py:827-846), fmt an OJX_FMT_* code: grad_x[M,K] = grad_y . Wdeq + v @ A^T, grad_a[K,rank]
+ * = x^T v and grad_b[rank,N] = u^T grad_y in dtype, with u = scaling * (x @ A) and v = scaling *
+ * (grad_y @ B^T) kept in fp32 in the caller's scratch lora_uv [2, M, rank].  Any of the three
+ * results may be null.  M, N, K >= 1.  The workspace (ojx_gemm_bwd_lora_workspace_bytes) holds
+ * the fp32 partial sums of row splits; a smaller one lowers the split counts. */
+int ojx_gemm_bwd_lora(int fmt, const void* x, const void* grad_y, const uint8_t* packed,
+                      const uint16_t* scales, const void* lora_a, const void* lora_b,
+                      int64_t rank, float scaling, float* lora_uv, void* grad_x, void* grad_a,
+                      void* grad_b, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype,
+                      void* workspace, size_t workspace_bytes, void* stream);
+int ojx_gemm_bwd_lora_workspace_bytes(int fmt, int64_t M, int64_t N, int64_t K, int64_t gs,
+                                      int64_t rank, int need_x, int need_a, int need_b, int dtype,
+                                      size_t* bytes);
+
 /* ---------------------------------------------------------------- 2-bit E8
  *
  * E8LatticePacker (2.0 bit/weight, ojasx2/math/lattice.py:209-279): four 2-bit codes per

@@ -290,7 +290,8 @@ static int gemm_fwd_lora(int fmt, const void* x, const uint8_t* packed, const ui
 // Backward dX of every format: grad_x[M, K] = grad_y[M, N] . Wdeq[N, K].
 static int gemm_bwd(int fmt, const void* grad_y, const uint8_t* packed, const uint16_t* scales,
                     void* grad_x, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype,
-                    void* ws, size_t ws_bytes, void* stream) {
+                    void* ws, size_t ws_bytes, void* stream,
+                    const ojx::LoraEp& lora = ojx::LoraEp{}) {
     if (int r = check_fmt_args(fmt, grad_y, packed, scales, grad_x, M, K, N, gs, dtype)) return r;
     if (int r = check_workspace(ws, ws_bytes)) return r;
     if (M == 0 || K == 0) return OJX_OK;
@@ -300,19 +301,67 @@ static int gemm_bwd(int fmt, const void* grad_y, const uint8_t* packed, const ui
     const Route route = route_bwd(fmt, grad_y, packed, scales, M, N, K, gs, dtype);
     if (route == kRouteMfma) {
         e = launch_mfma(grad_y, packed, scales, nullptr, grad_x, M, N, K, gs, dtype, s, fmt, true,
-                        ws, ws_bytes);
+                        ws, ws_bytes, lora);
     } else if (route == kRouteF32) {
         int splits = ojx::gemm_f32_bwd_splits(M, N, K);
         const size_t per = (size_t)ojx::split_stride(M, K) * sizeof(float);
         const size_t fit = ws ? ws_bytes / per : 0;
         if ((size_t)splits > fit) splits = fit < 2 ? 1 : (int)fit;
         e = ojx::launch_gemm_f32_bwd(grad_y, packed, scales, grad_x, static_cast<float*>(ws),
-                                     splits, M, N, K, gs, dtype, s, fmt);
-    } else
+                                     splits, M, N, K, gs, dtype, s, fmt, lora);
+    } else {
         e = ojx::launch_gemm_generic_bwd(grad_y, packed, scales, grad_x, M, N, K, gs, dtype, s,
-                                         fmt);
+                                         fmt, lora);
+    }
     if (e != hipSuccess) return fail(OJX_EHIP, "%s gemm_bwd_dx launch: %s", fmt_name(fmt),
                                      hipGetErrorString(e));
+    g_last_error[0] = '\0';
+    return OJX_OK;
+}
+
+// Backward of a linear with a LoRA adapter, after gemm_fwd_lora's forward: v = scaling *
+// (gy @ B^T) and u = scaling * (x @ A) in fp32 (one launch), grad_x = gy . W + v @ A^T (the
+// adapter term in the backward GEMM's epilogue), grad_a = x^T v, grad_b = u^T gy.
+static int gemm_bwd_lora(int fmt, const void* x, const void* grad_y, const uint8_t* packed,
+                         const uint16_t* scales, const void* lora_a, const void* lora_b,
+                         int64_t rank, float scaling, float* lora_uv, void* grad_x, void* grad_a,
+                         void* grad_b, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype,
+                         void* ws, size_t ws_bytes, void* stream) {
+    if (fmt != ojx::kFmtTernary && fmt != ojx::kFmt2Bit && fmt != ojx::kFmtRoot)
+        return fail(OJX_EINVAL, "unknown format code %d", fmt);
+    if (rank < 1 || rank > ojx::kLoraMaxRank)
+        return fail(OJX_ELAYOUT, "LoRA rank must be in 1..%lld (got %lld)",
+                    (long long)ojx::kLoraMaxRank, (long long)rank);
+    if (M < 1 || N < 1 || K < 1)
+        return fail(OJX_EINVAL, "adapter gradients need M, N, K >= 1 (M=%lld N=%lld K=%lld)",
+                    (long long)M, (long long)N, (long long)K);
+    if (!x || !grad_y || !packed || !scales || !lora_a || !lora_b || !lora_uv)
+        return fail(OJX_EINVAL, "null input pointer");
+    if (((uintptr_t)lora_uv & 3u) || ((uintptr_t)lora_a & 1u) || ((uintptr_t)lora_b & 1u))
+        return fail(OJX_ELAYOUT, "misaligned LoRA operand (lora_uv 4-byte, A and B 2-byte)");
+    if (int r = check_fmt_args(fmt, grad_y, packed, scales, grad_x ? grad_x : lora_uv, M, K, N, gs,
+                               dtype))
+        return r;
+    if (int r = check_workspace(ws, ws_bytes)) return r;
+    if (int r = check_device()) return r;
+    hipStream_t s = (hipStream_t)stream;
+    float *u = lora_uv, *v = lora_uv + M * rank;
+    hipError_t e = ojx::launch_lora_uv(x, grad_y, lora_a, lora_b, scaling, M, N, K, rank, dtype,
+                                       grad_b ? u : nullptr, grad_x || grad_a ? v : nullptr, s);
+    if (e != hipSuccess) return fail(OJX_EHIP, "lora_uv launch: %s", hipGetErrorString(e));
+    if (grad_x) {
+        // B[j, n] of the epilogue is A[k, j]: rank stride 1, column stride rank
+        ojx::LoraEp ep{v, lora_a, rank, rank, 1};
+        ep.ldn = rank;
+        if (int r = gemm_bwd(fmt, grad_y, packed, scales, grad_x, M, N, K, gs, dtype, ws, ws_bytes,
+                             stream, ep))
+            return r;
+    }
+    if (grad_a || grad_b) {
+        e = ojx::launch_lora_grads(x, grad_y, u, v, M, N, K, rank, dtype, grad_a, grad_b,
+                                   static_cast<float*>(ws), ws_bytes, s);
+        if (e != hipSuccess) return fail(OJX_EHIP, "lora_grads launch: %s", hipGetErrorString(e));
+    }
     g_last_error[0] = '\0';
     return OJX_OK;
 }
@@ -797,6 +846,31 @@ __attribute__((visibility("default"))) int ojx_e8r_gemm_bwd_dx(
     void* stream) {
     return gemm_bwd(ojx::kFmtRoot, grad_y, codes, scales, grad_x, M, N, K, gs, dtype, workspace,
                     workspace_bytes, stream);
+}
+
+// ---------------------------------------------------------------- adapter gradients
+
+__attribute__((visibility("default"))) int ojx_gemm_bwd_lora(
+    int fmt, const void* x, const void* grad_y, const uint8_t* packed, const uint16_t* scales,
+    const void* lora_a, const void* lora_b, int64_t rank, float scaling, float* lora_uv,
+    void* grad_x, void* grad_a, void* grad_b, int64_t M, int64_t N, int64_t K, int64_t gs,
+    int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+    return gemm_bwd_lora(fmt, x, grad_y, packed, scales, lora_a, lora_b, rank, scaling, lora_uv,
+                         grad_x, grad_a, grad_b, M, N, K, gs, dtype, workspace, workspace_bytes,
+                         stream);
+}
+
+__attribute__((visibility("default"))) int ojx_gemm_bwd_lora_workspace_bytes(
+    int fmt, int64_t M, int64_t N, int64_t K, int64_t gs, int64_t rank, int need_x, int need_a,
+    int need_b, int dtype, size_t* bytes) {
+    if (rank < 1 || rank > ojx::kLoraMaxRank)
+        return fail(OJX_ELAYOUT, "LoRA rank must be in 1..%lld (got %lld)",
+                    (long long)ojx::kLoraMaxRank, (long long)rank);
+    if (int r = workspace_bytes(fmt, 1, M, N, K, gs, dtype, bytes)) return r;
+    if (!need_x) *bytes = 0;
+    const size_t g = ojx::lora_grads_bytes(M, N, K, rank, need_a != 0, need_b != 0);
+    if (g > *bytes) *bytes = g;
+    return OJX_OK;
 }
 
 // ---------------------------------------------------------------- Hadamard rotation

@@ -41,9 +41,9 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float f) {
 }
 
 template <int DT> struct Elem;
-template <> struct Elem<kF32> { using T = float; };
-template <> struct Elem<kF16> { using T = uint16_t; };
-template <> struct Elem<kBF16> { using T = uint16_t; };
+template <> struct Elem<kF32> { using T = float; using Bits = uint32_t; };
+template <> struct Elem<kF16> { using T = uint16_t; using Bits = uint16_t; };
+template <> struct Elem<kBF16> { using T = uint16_t; using Bits = uint16_t; };
 
 template <int DT> __device__ __forceinline__ float load_as_f32(const void* p, int64_t i) {
     if constexpr (DT == kF32) return ((const float*)p)[i];

@@ -30,6 +30,7 @@
 // 9e-7 -> 3e-7 (2-norm): each wave's chain is a fraction of K.
 
 #include "e8t_device.h"
+#include "e8t_f32.h"
 #include "e8t_internal.h"
 #include "e8t_lut.h"
 #include "e8t_root.h"
@@ -98,47 +99,6 @@ __device__ __forceinline__ void decode8(const float4* tab, uint32_t code, float 
             else w[j] = bf16_bits_to_f32(bf16_bits_hw(w[j]));
         }
     }
-}
-
-__device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// n consecutive activations as loaded (fp32: n words, 16-bit: n / 2 words).
-template <int DT, int n> struct RawX {
-    static constexpr int W = DT == kF32 ? n : n / 2;
-    uint32_t w[W];
-
-    // byte offset vo; kNoRecordOffset (or any offset past the buffer) reads zeros
-    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, uint32_t vo) {
-        if constexpr (W % 4 == 0) {
-#pragma unroll
-            for (int i = 0; i < W / 4; ++i) {
-                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, vo + 16u * i, 0, 0);
-                w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
-            }
-        } else {
-            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(b, vo, 0, 0);
-            w[0] = v.x; w[1] = v.y;
-        }
-    }
-    __device__ __forceinline__ float get(int j) const {
-        if constexpr (DT == kF32) return __uint_as_float(w[j]);
-        const uint32_t h = (w[j / 2] >> (16 * (j & 1))) & 0xFFFFu;
-        return DT == kF16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
-    }
-};
-
-template <int DT> constexpr uint32_t esize() { return DT == kF32 ? 4 : 2; }
-
-// Buffer over `rows` rows of a row-major [M, width] matrix from row m0 (fewer at its end).
-template <int DT>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const void* a, int64_t m0, int64_t M,
-                                                              int64_t width, int rows) {
-    const int64_t left = M - m0 < rows ? M - m0 : rows;
-    return __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(static_cast<const char*>(a) + m0 * width * esize<DT>()), (short)0,
-        (int)(left * width * esize<DT>()), kRsrcWord3);
 }
 
 }  // namespace
@@ -491,7 +451,7 @@ template <int FMT, int DT, int MT, int NW, bool VEC>
 __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_bwd(
     const void* __restrict__ gy, const uint8_t* __restrict__ packed,
     const uint16_t* __restrict__ scales, void* __restrict__ gx, float* __restrict__ part,
-    int64_t M, int64_t N, int64_t K, int gs_shift) {
+    int64_t M, int64_t N, int64_t K, int gs_shift, LoraEp lora) {
     __shared__ float4 tab[quad_entries<FMT>()];
     __shared__ f32x4 red[NW / 2][MT * 8][64];
     const int lane = threadIdx.x & 63;
@@ -614,7 +574,11 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_bwd(
         }
         __syncthreads();
     }
-    if (wave != 0 || c >= codes) return;
+    if (wave != 0) return;
+    if (lora.r > 0)
+        lora_add<DT, MT, 8>(acc, lora, m0, M, K, lane, [&](int j) { return 8 * (int64_t)c + j; },
+                            blockIdx.z, gridDim.z);
+    if (c >= codes) return;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
 #pragma unroll
@@ -728,15 +692,16 @@ static hipError_t launch_f32_fwd_t(const void* x, const uint8_t* packed, const u
 template <int FMT, int DT, int MT, int NW>
 static hipError_t launch_f32_bwd_cfg(const void* gy, const uint8_t* packed,
                                      const uint16_t* scales, void* gx, float* part, int splits,
-                                     int64_t M, int64_t N, int64_t K, int sh, hipStream_t s) {
+                                     int64_t M, int64_t N, int64_t K, int sh, hipStream_t s,
+                                     const LoraEp& lora) {
     const dim3 grid((unsigned)((K + 127) / 128), (unsigned)((M + 16 * MT - 1) / (16 * MT)),
                     (unsigned)splits);
     if (N % 4 == 0 && ((uintptr_t)gy & (DT == kF32 ? 15u : 7u)) == 0)
         hipLaunchKernelGGL((gemm_f32_bwd<FMT, DT, MT, NW, true>), grid, dim3(64 * NW), 0, s, gy,
-                           packed, scales, gx, part, M, N, K, sh);
+                           packed, scales, gx, part, M, N, K, sh, lora);
     else
         hipLaunchKernelGGL((gemm_f32_bwd<FMT, DT, MT, NW, false>), grid, dim3(64 * NW), 0, s, gy,
-                           packed, scales, gx, part, M, N, K, sh);
+                           packed, scales, gx, part, M, N, K, sh, lora);
     const hipError_t e = hipGetLastError();
     if (splits == 1 || e != hipSuccess) return e;
     return launch_split_reduce(part, splits, nullptr, gx, M, K, DT, s);
@@ -745,17 +710,17 @@ static hipError_t launch_f32_bwd_cfg(const void* gy, const uint8_t* packed,
 template <int FMT, int DT>
 static hipError_t launch_f32_bwd_t(const void* gy, const uint8_t* packed, const uint16_t* scales,
                                    void* gx, float* part, int splits, int64_t M, int64_t N,
-                                   int64_t K, int sh, hipStream_t s) {
+                                   int64_t K, int sh, hipStream_t s, const LoraEp& lora) {
     switch (f32_row_tiles(M)) {
     case 1:
         return launch_f32_bwd_cfg<FMT, DT, 1, kF32BwdWaves>(gy, packed, scales, gx, part, splits, M,
-                                                            N, K, sh, s);
+                                                            N, K, sh, s, lora);
     case 2:
         return launch_f32_bwd_cfg<FMT, DT, 2, kF32BwdWaves>(gy, packed, scales, gx, part, splits, M,
-                                                            N, K, sh, s);
+                                                            N, K, sh, s, lora);
     default:
         return launch_f32_bwd_cfg<FMT, DT, 4, kF32BwdWaves / 2>(gy, packed, scales, gx, part,
-                                                                splits, M, N, K, sh, s);
+                                                                splits, M, N, K, sh, s, lora);
     }
 }
 
@@ -778,14 +743,14 @@ static hipError_t f32_fwd_fmt(const void* x, const uint8_t* packed, const uint16
 template <int FMT>
 static hipError_t f32_bwd_fmt(const void* gy, const uint8_t* packed, const uint16_t* scales,
                               void* gx, float* part, int splits, int64_t M, int64_t N, int64_t K,
-                              int sh, int dt, hipStream_t s) {
+                              int sh, int dt, hipStream_t s, const LoraEp& lora) {
     switch (dt) {
     case kF32:
-        return launch_f32_bwd_t<FMT, kF32>(gy, packed, scales, gx, part, splits, M, N, K, sh, s);
+        return launch_f32_bwd_t<FMT, kF32>(gy, packed, scales, gx, part, splits, M, N, K, sh, s, lora);
     case kF16:
-        return launch_f32_bwd_t<FMT, kF16>(gy, packed, scales, gx, part, splits, M, N, K, sh, s);
+        return launch_f32_bwd_t<FMT, kF16>(gy, packed, scales, gx, part, splits, M, N, K, sh, s, lora);
     default:
-        return launch_f32_bwd_t<FMT, kBF16>(gy, packed, scales, gx, part, splits, M, N, K, sh, s);
+        return launch_f32_bwd_t<FMT, kBF16>(gy, packed, scales, gx, part, splits, M, N, K, sh, s, lora);
     }
 }
 
@@ -802,13 +767,13 @@ hipError_t launch_gemm_f32_fwd(const void* x, const uint8_t* packed, const uint1
 
 hipError_t launch_gemm_f32_bwd(const void* gy, const uint8_t* packed, const uint16_t* scales,
                                void* gx, float* part, int splits, int64_t M, int64_t N, int64_t K,
-                               int64_t gs, int dt, hipStream_t s, int fmt) {
+                               int64_t gs, int dt, hipStream_t s, int fmt, const LoraEp& lora) {
     const int sh = log2_of(gs);
     if (fmt == kFmtRoot)
-        return f32_bwd_fmt<kFmtRoot>(gy, packed, scales, gx, part, splits, M, N, K, sh, dt, s);
+        return f32_bwd_fmt<kFmtRoot>(gy, packed, scales, gx, part, splits, M, N, K, sh, dt, s, lora);
     if (fmt == kFmt2Bit)
-        return f32_bwd_fmt<kFmt2Bit>(gy, packed, scales, gx, part, splits, M, N, K, sh, dt, s);
-    return f32_bwd_fmt<kFmtTernary>(gy, packed, scales, gx, part, splits, M, N, K, sh, dt, s);
+        return f32_bwd_fmt<kFmt2Bit>(gy, packed, scales, gx, part, splits, M, N, K, sh, dt, s, lora);
+    return f32_bwd_fmt<kFmtTernary>(gy, packed, scales, gx, part, splits, M, N, K, sh, dt, s, lora);
 }
 
 }  // namespace ojx

@@ -85,7 +85,7 @@ template <int FMT, int DT>
 __global__ __launch_bounds__(256) void gemm_generic_bwd(
     const void* __restrict__ gy, const uint8_t* __restrict__ packed,
     const uint16_t* __restrict__ scales, void* __restrict__ gx, int64_t M, int64_t N, int64_t K,
-    int64_t gs) {
+    int64_t gs, LoraEp lora) {
     __shared__ float gs_tile[kChunk][kTile + 4];  // [n][m]
     __shared__ float ws[kChunk][kTile + 4];       // [n][k]
     const int tid = threadIdx.x;
@@ -129,7 +129,8 @@ __global__ __launch_bounds__(256) void gemm_generic_bwd(
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int64_t gk = k0 + tk * 4 + j;
-            if (gk < K) store_from_f32<DT>(gx, gm * K + gk, acc[i][j]);
+            if (gk < K)
+                store_from_f32<DT>(gx, gm * K + gk, acc[i][j] + lora_term<DT>(lora, gm, gk));
         }
     }
 }
@@ -146,10 +147,11 @@ static hipError_t fwd_t(const void* x, const uint8_t* packed, const uint16_t* sc
 
 template <int FMT, int DT>
 static hipError_t bwd_t(const void* gy, const uint8_t* packed, const uint16_t* scales, void* gx,
-                        int64_t M, int64_t N, int64_t K, int64_t gs, hipStream_t stream) {
+                        int64_t M, int64_t N, int64_t K, int64_t gs, hipStream_t stream,
+                        const LoraEp& lora) {
     dim3 grid((unsigned)((K + kTile - 1) / kTile), (unsigned)((M + kTile - 1) / kTile));
     hipLaunchKernelGGL((gemm_generic_bwd<FMT, DT>), grid, dim3(256), 0, stream, gy, packed, scales,
-                       gx, M, N, K, gs);
+                       gx, M, N, K, gs, lora);
     return hipGetLastError();
 }
 
@@ -167,11 +169,11 @@ static hipError_t fwd_fmt(const void* x, const uint8_t* packed, const uint16_t* 
 template <int FMT>
 static hipError_t bwd_fmt(const void* gy, const uint8_t* packed, const uint16_t* scales, void* gx,
                           int64_t M, int64_t N, int64_t K, int64_t gs, int dt,
-                          hipStream_t stream) {
+                          hipStream_t stream, const LoraEp& lora) {
     switch (dt) {
-        case kF32: return bwd_t<FMT, kF32>(gy, packed, scales, gx, M, N, K, gs, stream);
-        case kF16: return bwd_t<FMT, kF16>(gy, packed, scales, gx, M, N, K, gs, stream);
-        default: return bwd_t<FMT, kBF16>(gy, packed, scales, gx, M, N, K, gs, stream);
+        case kF32: return bwd_t<FMT, kF32>(gy, packed, scales, gx, M, N, K, gs, stream, lora);
+        case kF16: return bwd_t<FMT, kF16>(gy, packed, scales, gx, M, N, K, gs, stream, lora);
+        default: return bwd_t<FMT, kBF16>(gy, packed, scales, gx, M, N, K, gs, stream, lora);
     }
 }
 
@@ -188,11 +190,11 @@ hipError_t launch_gemm_generic_fwd(const void* x, const uint8_t* packed, const u
 
 hipError_t launch_gemm_generic_bwd(const void* gy, const uint8_t* packed, const uint16_t* scales,
                                    void* gx, int64_t M, int64_t N, int64_t K, int64_t gs, int dt,
-                                   hipStream_t stream, int fmt) {
-    if (fmt == kFmtRoot) return bwd_fmt<kFmtRoot>(gy, packed, scales, gx, M, N, K, gs, dt, stream);
+                                   hipStream_t stream, int fmt, const LoraEp& lora) {
+    if (fmt == kFmtRoot) return bwd_fmt<kFmtRoot>(gy, packed, scales, gx, M, N, K, gs, dt, stream, lora);
     return fmt == kFmt2Bit
-               ? bwd_fmt<kFmt2Bit>(gy, packed, scales, gx, M, N, K, gs, dt, stream)
-               : bwd_fmt<kFmtTernary>(gy, packed, scales, gx, M, N, K, gs, dt, stream);
+               ? bwd_fmt<kFmt2Bit>(gy, packed, scales, gx, M, N, K, gs, dt, stream, lora)
+               : bwd_fmt<kFmtTernary>(gy, packed, scales, gx, M, N, K, gs, dt, stream, lora);
 }
 
 }  // namespace ojx

@@ -66,7 +66,8 @@ hipError_t launch_gemm_generic_fwd(const void* x, const uint8_t* packed, const u
                                    const LoraEp& lora = LoraEp{});
 hipError_t launch_gemm_generic_bwd(const void* gy, const uint8_t* packed, const uint16_t* scales,
                                    void* gx, int64_t M, int64_t N, int64_t K, int64_t gs, int dt,
-                                   hipStream_t stream, int fmt = 0);
+                                   hipStream_t stream, int fmt = 0,
+                                   const LoraEp& lora = LoraEp{});
 
 // The fused linear on the fp32 matrix instruction: every dtype, any M and N, rows of whole
 // scale groups (K % gs == 0) of 2^t >= 8 weights.  The backward's row splits (fp32 partial
@@ -81,7 +82,8 @@ hipError_t launch_gemm_f32_fwd(const void* x, const uint8_t* packed, const uint1
                                const LoraEp& lora);
 hipError_t launch_gemm_f32_bwd(const void* gy, const uint8_t* packed, const uint16_t* scales,
                                void* gx, float* part, int splits, int64_t M, int64_t N, int64_t K,
-                               int64_t gs, int dt, hipStream_t stream, int fmt);
+                               int64_t gs, int dt, hipStream_t stream, int fmt,
+                               const LoraEp& lora = LoraEp{});
 
 // y[M, N] = the sum of `splits` fp32 partial results (split_stride(M, N) apart) + bias,
 // rounded once to dtype.
@@ -222,6 +224,19 @@ struct LoraDown {
 constexpr int kLoraDownItems = 4;
 hipError_t launch_lora_down(const void* x, int64_t M, int64_t K, int dt, const LoraDown* items,
                             int n, hipStream_t stream);
+
+// The adapter gradients of a linear: A's [K, r] = x^T v and B's [r, N] = u^T gy for u = scaling *
+// (x @ A) and v = scaling * (gy @ B^T), fp32 [M, r] each.
+//   launch_lora_uv: u and / or v (either null to skip it), one launch;
+//   launch_lora_grads: grad_a and / or grad_b in dtype; row splits of the sums over M leave
+//   fp32 partials, lora_grads_bytes in all, in `part` (smaller or null: one split).
+hipError_t launch_lora_uv(const void* x, const void* gy, const void* a, const void* b,
+                          float scaling, int64_t M, int64_t N, int64_t K, int64_t r, int dt,
+                          float* u, float* v, hipStream_t stream);
+size_t lora_grads_bytes(int64_t M, int64_t N, int64_t K, int64_t r, bool need_a, bool need_b);
+hipError_t launch_lora_grads(const void* x, const void* gy, const float* u, const float* v,
+                             int64_t M, int64_t N, int64_t K, int64_t r, int dt, void* grad_a,
+                             void* grad_b, float* part, size_t part_bytes, hipStream_t stream);
 
 // Records `msg` as the calling thread's last error (ojx_e8t_last_error) and returns `code`.
 int api_fail(int code, const char* msg);

@@ -32,6 +32,8 @@ EXPORTS = (
     "ojx_e8_gemm_fwd_lora",
     "ojx_e8r_gemm_fwd_lora",
     "ojx_e8t_gemm_bwd_dx",
+    "ojx_gemm_bwd_lora",
+    "ojx_gemm_bwd_lora_workspace_bytes",
     "ojx_e8t_gemv_grouped_plan",
     "ojx_e8t_gemv_grouped",
     "ojx_e8_gemv_grouped_plan",
@@ -122,6 +124,12 @@ def lib() -> ctypes.CDLL:
                 fn.restype = _INT
                 fn.argtypes = [_P, _P, _P, _P, _P, _P, _I64, _F32, _P, _P, _I64, _I64, _I64,
                                _I64, _INT, _P, _SZ, _P]
+            L.ojx_gemm_bwd_lora.restype = _INT
+            L.ojx_gemm_bwd_lora.argtypes = [_INT, _P, _P, _P, _P, _P, _P, _I64, _F32, _P, _P, _P,
+                                            _P, _I64, _I64, _I64, _I64, _INT, _P, _SZ, _P]
+            L.ojx_gemm_bwd_lora_workspace_bytes.restype = _INT
+            L.ojx_gemm_bwd_lora_workspace_bytes.argtypes = [_INT, _I64, _I64, _I64, _I64, _I64,
+                                                            _INT, _INT, _INT, _INT, _P]
             L.ojx_e8t_gemm_bwd_dx.restype = _INT
             L.ojx_e8t_gemm_bwd_dx.argtypes = [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _INT, _P,
                                              _SZ, _P]

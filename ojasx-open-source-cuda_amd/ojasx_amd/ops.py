@@ -336,28 +336,83 @@ def _linear_lora_setup_context(ctx, inputs, output):
     ctx.bias_dtype = None if bias is None else bias.dtype
 
 
+@torch.library.custom_op(f"{_NS}::linear_lora_bwd", mutates_args=())
+def linear_lora_bwd(x: torch.Tensor, grad_y: torch.Tensor, packed_weight: torch.Tensor,
+                    block_scales: torch.Tensor, lora_a: torch.Tensor, lora_b: torch.Tensor,
+                    scaling: float, fmt: int, out_features: int, in_features: int,
+                    group_size: int, need_x: bool, need_a: bool, need_b: bool
+                    ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Gradients of linear_lora for x, lora_a and lora_b (those not needed come back empty):
+    the adapter products in fp32, grad_x with the adapter term added in the backward GEMM's
+    epilogue.  Every operand in grad_y's dtype, at least one row."""
+    dev = N.require_device(x, grad_y, packed_weight, block_scales, lora_a, lora_b)
+    dt = _dtype_code(grad_y.dtype)
+    x2 = x.reshape(-1, in_features).contiguous()
+    gy = grad_y.reshape(-1, out_features).contiguous()
+    la, lb = lora_a.contiguous(), lora_b.contiguous()
+    M, r = gy.shape[0], la.shape[1]
+    pw = packed_weight.contiguous()
+    bs = block_scales.to(torch.float16).contiguous()
+    gx = torch.empty((M if need_x else 0, in_features), dtype=gy.dtype, device=dev)
+    ga = torch.empty((in_features, r) if need_a else (0, r), dtype=gy.dtype, device=dev)
+    gb = torch.empty((r, out_features) if need_b else (r, 0), dtype=gy.dtype, device=dev)
+    uv = torch.empty((2, M, r), dtype=torch.float32, device=dev)
+    with torch.cuda.device(dev):
+        nbytes = ctypes.c_size_t(0)
+        N.check(N.lib().ojx_gemm_bwd_lora_workspace_bytes(
+            fmt, M, out_features, in_features, group_size, r, int(need_x), int(need_a),
+            int(need_b), dt, ctypes.byref(nbytes)), "gemm_bwd_lora_workspace_bytes")
+        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dev) if nbytes.value else None
+        N.check(N.lib().ojx_gemm_bwd_lora(
+            fmt, N.ptr(x2), N.ptr(gy), N.ptr(pw), N.ptr(bs), N.ptr(la), N.ptr(lb), r,
+            float(scaling), N.ptr(uv), N.ptr(gx) if need_x else 0, N.ptr(ga) if need_a else 0,
+            N.ptr(gb) if need_b else 0, M, out_features, in_features, group_size, dt, N.ptr(ws),
+            nbytes.value, N.stream_handle(dev)), "gemm_bwd_lora")
+    return gx, ga, gb
+
+
+@linear_lora_bwd.register_fake
+def _(x, grad_y, packed_weight, block_scales, lora_a, lora_b, scaling, fmt, out_features,
+      in_features, group_size, need_x, need_a, need_b):
+    rows, r = grad_y.numel() // out_features, lora_a.shape[1]
+    return (grad_y.new_empty((rows if need_x else 0, in_features)),
+            grad_y.new_empty((in_features, r) if need_a else (0, r)),
+            grad_y.new_empty((r, out_features) if need_b else (r, 0)))
+
+
 def _linear_lora_backward(ctx, grad_y):
-    """grad_x through the fused backward dX plus the adapter's term; the adapter's own
-    gradients (and the bias's) in torch, as the reference computes them."""
+    """grad_x through the fused backward dX plus the adapter's term, and the adapter's own
+    gradients: one fused op, or torch products where the gradients themselves are to be
+    differentiated (create_graph) or there are no rows; the bias's gradient in torch."""
     x, packed_weight, block_scales, lora_a, lora_b = ctx.saved_tensors
     out_features, in_features, group_size = ctx.dims
     sc = ctx.scaling
+    need_x, need_a, need_b = (ctx.needs_input_grad[i] for i in (0, 4, 5))
     gy = grad_y.reshape(-1, out_features).contiguous()
-    x2 = x.reshape(-1, in_features)
     la = lora_a.to(grad_y.dtype)
     lb = lora_b.to(grad_y.dtype)
-    gyb = gy @ lb.t().contiguous()                       # [M, r]
     grad_x = grad_a = grad_b = grad_bias = None
-    if ctx.needs_input_grad[0]:
+    if ctx.has_bias and ctx.needs_input_grad[3]:
+        grad_bias = gy.sum(dim=0).to(ctx.bias_dtype)
+    if not torch.is_grad_enabled() and gy.shape[0] > 0 and x.dtype == gy.dtype:
+        if need_x or need_a or need_b:
+            gx, ga, gb = linear_lora_bwd(x, gy, packed_weight, block_scales, la, lb, sc, ctx.fmt,
+                                         out_features, in_features, group_size, need_x, need_a,
+                                         need_b)
+            grad_x = gx.reshape(x.shape) if need_x else None
+            grad_a = ga.to(lora_a.dtype) if need_a else None
+            grad_b = gb.to(lora_b.dtype) if need_b else None
+        return grad_x, None, None, grad_bias, grad_a, grad_b, None, None, None, None, None
+    x2 = x.reshape(-1, in_features)
+    gyb = gy @ lb.t().contiguous()                       # [M, r]
+    if need_x:
         grad_x = _linear_bwd(ctx.fmt, gy, packed_weight, block_scales, out_features,
                              in_features, group_size)
         grad_x = (grad_x + sc * (gyb @ la.t().contiguous())).reshape(x.shape)
-    if ctx.needs_input_grad[4]:
+    if need_a:
         grad_a = (sc * (x2.t().contiguous() @ gyb)).to(lora_a.dtype)
-    if ctx.needs_input_grad[5]:
+    if need_b:
         grad_b = (sc * ((x2 @ la).t().contiguous() @ gy)).to(lora_b.dtype)
-    if ctx.has_bias and ctx.needs_input_grad[3]:
-        grad_bias = gy.sum(dim=0).to(ctx.bias_dtype)
     return grad_x, None, None, grad_bias, grad_a, grad_b, None, None, None, None, None
 
 

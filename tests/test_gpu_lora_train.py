@@ -74,3 +74,61 @@ def test_forward(fmt, M, N, K, gs, r, dtype):
     ref = x @ w.t() + s * (x @ a) @ b + bias
     mag = x.abs() @ w.abs().t() + s * (x.abs() @ a.abs()) @ b.abs() + bias.abs()
     _check(y, ref, mag, K + r, dtype, "forward")
+
+
+def _grads(t, pk, sc, s, fmt, N, K, gs, need=("x", "a", "b"), **kw):
+    d = {k: v.to(DEV).requires_grad_(k in need) for k, v in t.items() if k not in ("gy", "bias")}
+    y = ops.linear_lora(d["x"], pk, sc, None, d["a"], d["b"], s, fmt, N, K, gs)
+    return torch.autograd.grad(y, [d[k] for k in need], t["gy"].to(DEV), **kw)
+
+
+@pytest.mark.parametrize("fmt,M,N,K,gs,r,dtype", SHAPES + [
+    (ops.FMT_TERNARY, 4100, 320, 256, 32, 12, bf16),   # row splits with fp32 partial sums
+    (ops.FMT_E8, 300, 100, 24, 24, 9, f16),            # the SIMT kernel (group size 24)
+])
+def test_gradients(fmt, M, N, K, gs, r, dtype):
+    t, pk, sc, w = _case(fmt, M, N, K, gs, r, dtype)
+    s = 0.5
+    print(f"lora bwd fmt={fmt} M={M} N={N} K={K} gs={gs} r={r} {dtype}", flush=True)
+    gx, ga, gb = _grads(t, pk, sc, s, fmt, N, K, gs)
+    x, a, b, gy = (t[k].double() for k in ("x", "a", "b", "gy"))
+    v, u = s * gy @ b.t(), s * x @ a
+    mv, mu = s * gy.abs() @ b.abs().t(), s * x.abs() @ a.abs()
+    _check(gx, gy @ w + v @ a.t(), gy.abs() @ w.abs() + mv @ a.abs().t(), 2 * N + r, dtype, "x")
+    _check(ga, x.t() @ v, x.abs().t() @ mv, N + M, dtype, "lora_a")
+    _check(gb, u.t() @ gy, mu.t() @ gy.abs(), K + M, dtype, "lora_b")
+
+
+@pytest.mark.parametrize("need", [("x",), ("a",), ("b",), ("a", "b"), ("x", "b")])
+def test_gradients_of_some(need):
+    """Frozen operands: the others' gradients are the ones of the full call, bit for bit."""
+    fmt, M, N, K, gs, r = ops.FMT_TERNARY, 1500, 256, 512, 32, 8
+    t, pk, sc, _ = _case(fmt, M, N, K, gs, r, bf16)
+    full = dict(zip(("x", "a", "b"), _grads(t, pk, sc, 2.0, fmt, N, K, gs)))
+    some = dict(zip(need, _grads(t, pk, sc, 2.0, fmt, N, K, gs, need=need)))
+    for k, v in some.items():
+        if k == "x" or len(need) > 1:
+            assert torch.equal(v, full[k])
+        else:  # one factor alone may split its rows differently: fp32 sums in another order
+            assert (v.float() - full[k].float()).abs().max() <= 2 ** -7 * full[k].float().abs().max()
+
+
+def test_gradients_other_callers():
+    """A transposed view of x, a batch of sequences, no rows, and gradients that are themselves
+    to be differentiated (these keep the torch products)."""
+    fmt, N, K, gs, r = ops.FMT_TERNARY, 96, 256, 32, 8
+    t, pk, sc, _ = _case(fmt, 24, N, K, gs, r, bf16)
+    ref = _grads(t, pk, sc, 2.0, fmt, N, K, gs)
+    view = dict(t, x=t["x"].t().contiguous().t())
+    assert all(torch.equal(p, q) for p, q in zip(ref, _grads(view, pk, sc, 2.0, fmt, N, K, gs)))
+    batch = dict(t, x=t["x"].view(4, 6, K), gy=t["gy"].view(4, 6, N))
+    out = _grads(batch, pk, sc, 2.0, fmt, N, K, gs)
+    assert out[0].shape == (4, 6, K)
+    assert all(torch.equal(p.reshape(q.shape), q) for p, q in zip(out, ref))
+    none = dict(t, x=t["x"][:0], gy=t["gy"][:0])
+    out = _grads(none, pk, sc, 2.0, fmt, N, K, gs)
+    assert out[0].shape == (0, K) and not out[1].any() and not out[2].any()
+    out = _grads(t, pk, sc, 2.0, fmt, N, K, gs, create_graph=True)
+    assert out[1].requires_grad and out[2].requires_grad
+    for p, q in zip(out, ref):  # three bf16 roundings more than the fused gradients
+        assert (p.float() - q.float()).abs().max() <= 2 ** -6 * q.float().abs().max()
