@@ -1,4 +1,4 @@
-"""Builds libojasx_e8t.so (HIP kernels + C ABI) for gfx950, in-tree.
+"""Builds libojasx_e8t.so (HIP kernels + C ABI) and _ojasx_eager.so for gfx950, in-tree.
 
     python ojasx-open-source-cuda_amd/build.py
 
@@ -18,6 +18,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "lib", "libojasx_e8t.so")
+# CPython extension of the eager calls (torch's C++ tensors over the C ABI), linked to LIB
+EAGER = os.path.join(HERE, "lib", "_ojasx_eager.so")
 
 SOURCES = [
     "e8t_codec.hip",
@@ -60,11 +62,52 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_eager() -> str:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    if not os.path.exists(os.path.join(rocm, "include", "hip", "hip_runtime.h")):
+        rocm = "/opt/rocm"
+    obj = os.path.join(BUILD, "e8t_torch.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for d in cpp_extension.include_paths() + [os.path.join(rocm, "include"),
+                                              sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", d]
+    r = subprocess.run(cmd + ["-c", os.path.join(CSRC, "e8t_torch.cpp"), "-o", obj],
+                       capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stdout + r.stderr)
+        raise RuntimeError("g++ failed for e8t_torch.cpp")
+    return obj
+
+
+def _link_eager(obj: str) -> None:
+    import torch
+
+    libdir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = EAGER + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, obj, f"-L{libdir}", f"-L{os.path.dirname(LIB)}",
+           "-l:libojasx_e8t.so", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+           "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN", "-Wl,--no-as-needed"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stdout + r.stderr)
+        raise RuntimeError("link of _ojasx_eager.so failed")
+    os.replace(tmp, EAGER)
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(BUILD, exist_ok=True)
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=8) as ex:
+        eager = ex.submit(_compile_eager)
         objs = list(ex.map(_compile, SOURCES))
+        eager_obj = eager.result()
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -81,6 +124,7 @@ def build(verbose: bool = False) -> str:
         if missing:
             raise RuntimeError("libojasx_e8t.so has undefined symbols: " + ", ".join(missing[:4]))
     os.replace(tmp, LIB)
+    _link_eager(eager_obj)
     if verbose:
         print("built", LIB)
     return LIB

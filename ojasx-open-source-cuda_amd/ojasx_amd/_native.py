@@ -15,6 +15,7 @@ import torch
 
 _PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG_ROOT, "lib", "libojasx_e8t.so")
+EAGER_PATH = os.path.join(_PKG_ROOT, "lib", "_ojasx_eager.so")
 
 F32, F16, BF16, F64 = 0, 1, 2, 3
 DTYPE_CODE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
@@ -177,6 +178,30 @@ def lib() -> ctypes.CDLL:
             L.ojx_e8_ste_quantize_dt.argtypes = [_P, _INT, _I64, _P, _P]
             _lib = L
     return _lib
+
+
+_eager = None
+
+
+def eager():
+    """The extension of the eager calls (csrc/e8t_torch.cpp).  Its functions return None for
+    every call that is not plain eager work on GPU tensors; the caller then takes the
+    registered op.  Not for code under torch.compile (check torch.compiler.is_compiling())."""
+    global _eager
+    if _eager is None:
+        import importlib.util
+
+        with _lock:
+            if _eager is None:
+                if not os.path.exists(EAGER_PATH):
+                    raise RuntimeError(
+                        f"ojasx_amd: {EAGER_PATH} is missing; build it with "
+                        "`python ojasx-open-source-cuda_amd/build.py` (hipcc, gfx950)")
+                spec = importlib.util.spec_from_file_location("_ojasx_eager", EAGER_PATH)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+                _eager = mod
+    return _eager
 
 
 def check(status: int, what: str) -> None:

@@ -43,6 +43,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _native as N
 from . import ops
 
 __all__ = [
@@ -225,6 +226,33 @@ def _get_ternary_e8_luts(device: Optional[torch.device] = None
     return _DEVICE_TERNARY_LUTS[key]
 
 
+# Code formats of the bitrates, and their registered ops.  Eager calls on plain GPU tensors go
+# through N.eager() instead, without the ops' dispatch (csrc/e8t_torch.cpp: one bf16 token
+# through a 4096 x 4096 layer takes 6.2 instead of 26.2 us).
+_FMT = {1.5: ops.FMT_TERNARY, 1.0: ops.FMT_ROOT}
+_ENCODE = {ops.FMT_TERNARY: ops.encode, ops.FMT_E8: ops.encode2, ops.FMT_ROOT: ops.encode1}
+_DECODE = {ops.FMT_TERNARY: ops.decode, ops.FMT_E8: ops.decode2, ops.FMT_ROOT: ops.decode1}
+
+
+def _fmt_of(bitrate: float) -> int:
+    return _FMT.get(bitrate, ops.FMT_E8)
+
+
+def _encode(w: torch.Tensor, group_size: int, fmt: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    out = None
+    if not torch.compiler.is_compiling():
+        out = N.eager().encode(w, group_size, fmt)
+    return _ENCODE[fmt](w, group_size) if out is None else out
+
+
+def _decode(packed: torch.Tensor, scales: torch.Tensor, numel: int, group_size: int,
+            dtype: torch.dtype, fmt: int) -> torch.Tensor:
+    out = None
+    if not torch.compiler.is_compiling() and dtype in N.DTYPE_CODE:
+        out = N.eager().decode(packed, scales, numel, group_size, N.DTYPE_CODE[dtype], fmt)
+    return _DECODE[fmt](packed, scales, numel, group_size, dtype) if out is None else out
+
+
 def _on_gpu(t: torch.Tensor) -> torch.Tensor:
     if t.device.type == "cuda":
         return t
@@ -242,7 +270,7 @@ class TernaryE8LatticePacker:
         m, n = w.shape
         if group_size <= 0 or group_size % 16 != 0:
             group_size = 16  # silent coercion, lattice.py:346-347
-        packed, scales = ops.encode(_on_gpu(w), group_size)
+        packed, scales = _encode(_on_gpu(w), group_size, ops.FMT_TERNARY)
         if w.device.type != "cuda":
             packed, scales = packed.to(w.device), scales.to(w.device)
         return packed, scales, (m, n)
@@ -256,8 +284,8 @@ class TernaryE8LatticePacker:
         total = shape[0] * shape[1]
         padded = (packed_codes.numel() // 3) * 16
         group_size = padded // max(1, scales.numel())  # inferred as in lattice.py:407-409
-        out = ops.decode(_on_gpu(packed_codes), _on_gpu(scales).to(torch.float16), total,
-                         group_size, dtype)
+        out = _decode(_on_gpu(packed_codes), _on_gpu(scales).to(torch.float16), total,
+                      group_size, dtype, ops.FMT_TERNARY)
         if packed_codes.device.type != "cuda":
             out = out.to(packed_codes.device)
         return out.view(shape)
@@ -272,7 +300,7 @@ class E8LatticePacker:
         m, n = w.shape
         if group_size <= 0 or group_size % 8 != 0:
             raise ValueError(f"group_size ({group_size}) must be a positive multiple of 8.")
-        packed, scales = ops.encode2(_on_gpu(w), group_size)
+        packed, scales = _encode(_on_gpu(w), group_size, ops.FMT_E8)
         if w.device.type != "cuda":
             packed, scales = packed.to(w.device), scales.to(w.device)
         return packed, scales, (m, n)
@@ -284,8 +312,8 @@ class E8LatticePacker:
         total = shape[0] * shape[1]
         padded = packed_codes.numel() * 4
         group_size = padded // max(1, scales.numel())  # inferred as in lattice.py:264-266
-        out = ops.decode2(_on_gpu(packed_codes), _on_gpu(scales).to(torch.float16), total,
-                          group_size, dtype)
+        out = _decode(_on_gpu(packed_codes), _on_gpu(scales).to(torch.float16), total,
+                      group_size, dtype, ops.FMT_E8)
         if packed_codes.device.type != "cuda":
             out = out.to(packed_codes.device)
         return out.view(shape)
@@ -337,7 +365,7 @@ class RootE8LatticePacker:
         m, n = w.shape
         if group_size <= 0 or group_size % 8 != 0:
             group_size = 8  # silent coercion, lattice.py:485-486
-        codes, scales = ops.encode1(_on_gpu(w), group_size)
+        codes, scales = _encode(_on_gpu(w), group_size, ops.FMT_ROOT)
         if w.device.type != "cuda":
             codes, scales = codes.to(w.device), scales.to(w.device)
         return codes, scales, (m, n)
@@ -349,8 +377,8 @@ class RootE8LatticePacker:
         total = shape[0] * shape[1]
         padded = packed_codes.numel() * 8
         group_size = padded // max(1, scales.numel())  # inferred as in lattice.py:524-525
-        out = ops.decode1(_on_gpu(packed_codes), _on_gpu(scales).to(torch.float16), total,
-                          group_size, dtype)
+        out = _decode(_on_gpu(packed_codes), _on_gpu(scales).to(torch.float16), total,
+                      group_size, dtype, ops.FMT_ROOT)
         if packed_codes.device.type != "cuda":
             out = out.to(packed_codes.device)
         return out.view(shape)
@@ -390,6 +418,11 @@ class _FusedE8GEMMFunction(torch.autograd.Function):
         ctx.x_shape = x_rot.shape
         ctx.has_bias = bias is not None
         ctx.use_hadamard = use_hadamard
+        if not torch.compiler.is_compiling():
+            y = N.eager().linear(x_rot, packed_weight, block_scales, bias, out_features,
+                                 in_features, group_size, _fmt_of(ctx.bitrate))
+            if y is not None:
+                return y
         linear = {1.5: ops.e8t_linear, 1.0: ops.e8r_linear}.get(ctx.bitrate, ops.e8_linear)
         return linear(x_rot, packed_weight, block_scales, bias, out_features, in_features,
                       group_size)
@@ -398,15 +431,35 @@ class _FusedE8GEMMFunction(torch.autograd.Function):
     def backward(ctx, grad_y):
         packed_weight, block_scales = ctx.saved_tensors
         out_features, in_features, group_size = ctx.dims
-        bwd = {1.5: ops.e8t_linear_bwd_dx, 1.0: ops.e8r_linear_bwd_dx}.get(
-            ctx.bitrate, ops.e8_linear_bwd_dx)
-        grad_x = bwd(grad_y.contiguous(), packed_weight, block_scales, out_features,
-                     in_features, group_size)
+        grad_x = None
+        if not torch.compiler.is_compiling():
+            grad_x = N.eager().linear_bwd(grad_y, packed_weight, block_scales, out_features,
+                                          in_features, group_size, _fmt_of(ctx.bitrate))
+        if grad_x is None:
+            bwd = {1.5: ops.e8t_linear_bwd_dx, 1.0: ops.e8r_linear_bwd_dx}.get(
+                ctx.bitrate, ops.e8_linear_bwd_dx)
+            grad_x = bwd(grad_y.contiguous(), packed_weight, block_scales, out_features,
+                         in_features, group_size)
         grad_x = grad_x.reshape(ctx.x_shape)
         if ctx.use_hadamard and in_features % 32 == 0:
             grad_x = fwht_block32(grad_x)
         grad_bias = grad_y.reshape(-1, out_features).sum(dim=0) if ctx.has_bias else None
         return grad_x, None, None, grad_bias, None, None, None, None, None
+
+
+class _LoraLinearFunction(torch.autograd.Function):
+    """linear_lora recorded for plain eager calls (the registered op's own autograd formula,
+    without its dispatch)."""
+
+    @staticmethod
+    def forward(ctx, *args):
+        ops._linear_lora_setup_context(ctx, args, None)
+        y = N.eager().linear_lora(*args)
+        return ops.linear_lora(*args) if y is None else y
+
+    @staticmethod
+    def backward(ctx, grad_y):
+        return ops._linear_lora_backward(ctx, grad_y)
 
 
 class E8LatticeLinear(nn.Module):
@@ -490,16 +543,29 @@ class E8LatticeLinear(nn.Module):
 
     def forward_fused(self, x: torch.Tensor) -> torch.Tensor:
         has_lora = self.rank > 0 and self.lora_A is not None and self.lora_B is not None
+        plain = not (self.use_hadamard or torch.compiler.is_compiling())
         if (has_lora and not self.use_hadamard and self.lora_A.shape[-1] <= ops.LORA_MAX_RANK
                 and x.is_cuda):
             # the adapter term scaling * ((x @ A) @ B) (lattice.py:839-842) added inside the
             # E8 kernel's epilogue; with a Hadamard rotation the E8 op sees the rotated x
             # while the adapter takes the original, so that case stays unfused below
             _require_supported(self.bitrate)
-            fmt = {1.5: ops.FMT_TERNARY, 1.0: ops.FMT_ROOT}.get(float(self.bitrate), ops.FMT_E8)
-            return ops.linear_lora(x, self.packed_weight, self.block_scales, self.bias,
-                                   self.lora_A, self.lora_B, float(self.scaling), fmt,
-                                   self.out_features, self.in_features, self.group_size)
+            args = (x, self.packed_weight, self.block_scales, self.bias, self.lora_A,
+                    self.lora_B, float(self.scaling), _fmt_of(float(self.bitrate)),
+                    self.out_features, self.in_features, self.group_size)
+            if plain:
+                y = N.eager().linear_lora(*args)  # None: gradients to record, or not plain
+                if y is not None:
+                    return y
+                if N.eager().is_plain(*args[:6]):
+                    return _LoraLinearFunction.apply(*args)
+            return ops.linear_lora(*args)
+        if plain and not has_lora:
+            y = N.eager().linear(x, self.packed_weight, self.block_scales, self.bias,
+                                 self.out_features, self.in_features, self.group_size,
+                                 _fmt_of(float(self.bitrate)))
+            if y is not None:
+                return y
         out = _FusedE8GEMMFunction.apply(x, self.packed_weight, self.block_scales, self.bias,
                                          self.out_features, self.in_features, self.group_size,
                                          self.bitrate, self.use_hadamard)

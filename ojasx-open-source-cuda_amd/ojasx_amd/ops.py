@@ -388,21 +388,28 @@ def _linear_lora_backward(ctx, grad_y):
     out_features, in_features, group_size = ctx.dims
     sc = ctx.scaling
     need_x, need_a, need_b = (ctx.needs_input_grad[i] for i in (0, 4, 5))
-    gy = grad_y.reshape(-1, out_features).contiguous()
     la = lora_a.to(grad_y.dtype)
     lb = lora_b.to(grad_y.dtype)
     grad_x = grad_a = grad_b = grad_bias = None
     if ctx.has_bias and ctx.needs_input_grad[3]:
-        grad_bias = gy.sum(dim=0).to(ctx.bias_dtype)
-    if not torch.is_grad_enabled() and gy.shape[0] > 0 and x.dtype == gy.dtype:
+        grad_bias = grad_y.reshape(-1, out_features).sum(dim=0).to(ctx.bias_dtype)
+    if not torch.is_grad_enabled() and grad_y.numel() > 0 and x.dtype == grad_y.dtype:
         if need_x or need_a or need_b:
-            gx, ga, gb = linear_lora_bwd(x, gy, packed_weight, block_scales, la, lb, sc, ctx.fmt,
-                                         out_features, in_features, group_size, need_x, need_a,
-                                         need_b)
+            out = None
+            if not torch.compiler.is_compiling():
+                out = N.eager().linear_lora_bwd(x, grad_y, packed_weight, block_scales, la, lb, sc,
+                                                ctx.fmt, out_features, in_features, group_size,
+                                                need_x, need_a, need_b)
+            if out is None:
+                out = linear_lora_bwd(x, grad_y, packed_weight, block_scales, la, lb, sc, ctx.fmt,
+                                      out_features, in_features, group_size, need_x, need_a,
+                                      need_b)
+            gx, ga, gb = out
             grad_x = gx.reshape(x.shape) if need_x else None
             grad_a = ga.to(lora_a.dtype) if need_a else None
             grad_b = gb.to(lora_b.dtype) if need_b else None
         return grad_x, None, None, grad_bias, grad_a, grad_b, None, None, None, None, None
+    gy = grad_y.reshape(-1, out_features).contiguous()
     x2 = x.reshape(-1, in_features)
     gyb = gy @ lb.t().contiguous()                       # [M, r]
     if need_x:
