@@ -352,76 +352,152 @@ hipError_t launch_encode(const void* w, int wdt, int64_t numel, int64_t gs, uint
     }
 }
 
-// ---------------------------------------------------------------- decoder
+// ---------------------------------------------------------------- decoders
+//
+// The three packers' unpack (lattice.py:386-419, 252-279, 519-533): coordinate *
+// scales.to(dtype), rounded to dtype for 2-bit and 1-bit codes.  Bound by the writes: a
+// lane writes 16 bytes (4 fp32 or 8 16-bit weights, half a code or one) of each of its
+// kDecPieces pieces, and a wave's store covers 1 KB without a gap.  One lane per 16 weights
+// left 64-byte gaps between the lanes of every store, and divided twice by the group size.
+// us for 14336 x 4096, gs 32, to fp32 / fp16 / bf16: ternary 71 / 24.5 / 29 -> 38 / 22.2 /
+// 22.7, 2-bit 71 / 24.5 / 29 -> 38 / 23 / 25, 1-bit 92 / 60 / 61 -> 39 / 24 / 24 (fp32: 6.4
+// TB/s written).
 
 constexpr int kDecThreads = 256;
+constexpr int kDecPieces = 4;
 
-template <int ODT>
-__global__ __launch_bounds__(kDecThreads) void decode_kernel(
-    const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales, int64_t numel,
-    int64_t gs, bool vec_ok, void* __restrict__ out) {
-    const int64_t p = (int64_t)blockIdx.x * kDecThreads + threadIdx.x;  // code pair
-    const int64_t e0 = p * 16;
-    if (e0 >= numel) return;
-    const uint32_t b0 = packed[3 * p], b1 = packed[3 * p + 1], b2 = packed[3 * p + 2];
-    uint32_t raw0 = 2u * (b0 | ((b1 & 0x0Fu) << 8));
-    uint32_t raw1 = 2u * ((b1 >> 4) | (b2 << 4));
-    const float s = scale_for<ODT>(scales[e0 / gs]);  // gs % 16 == 0: one group per pair
-    float v[16];
+// Bits of v in dtype ODT, rounded once (v kept a rounded fp32 product: -1 * 0 stays -0).
+template <int ODT> __device__ __forceinline__ uint32_t out_bits(float v) {
+    keep_f32(v);
+    if constexpr (ODT == kF32) return __float_as_uint(v);
+    else if constexpr (ODT == kF16) return f32_to_f16_bits(v);
+    else return f32_to_bf16_bits(v);
+}
+
+// FMT's weights e .. e + V - 1 (one code, or one half of it; one scale group) as bits of ODT.
+// Ternary and 2-bit weights take one of three or four values per group: each is rounded
+// once and selected by digit (digits by 24-bit multiplies; the compiler's division by 3
+// multiplies at a quarter of the rate).
+template <int FMT, int ODT, int V>
+__device__ __forceinline__ void decode_run(const uint8_t* __restrict__ packed, int64_t e,
+                                           uint32_t s16, uint32_t (&v)[V]) {
+    const float s = scale_for<ODT>(s16);
+    if constexpr (FMT == kFmt2Bit) {
+        uint32_t bits = packed[e >> 2];
+        if constexpr (V == 8) bits |= (uint32_t)packed[(e >> 2) + 1] << 8;
+        const uint32_t v0 = out_bits<ODT>(-1.5f * s), v1 = out_bits<ODT>(-0.5f * s),
+                       v2 = out_bits<ODT>(0.5f * s), v3 = out_bits<ODT>(1.5f * s);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        v[i] = (float)((int)(raw0 % 3u) - 1) * s;
-        v[8 + i] = (float)((int)(raw1 % 3u) - 1) * s;
-        keep_f32(v[i]);  // -1 * 0 stays -0 (see keep_f32)
-        keep_f32(v[8 + i]);
-        raw0 /= 3u;
-        raw1 /= 3u;
-    }
-    if (vec_ok && e0 + 16 <= numel) {
-        if constexpr (ODT == kF32) {
-            float4* o = reinterpret_cast<float4*>((float*)out + e0);
+        for (int i = 0; i < V; ++i) {
+            const uint32_t lo = (bits >> (2 * i)) & 1u ? v1 : v0;
+            const uint32_t hi = (bits >> (2 * i)) & 1u ? v3 : v2;
+            v[i] = (bits >> (2 * i)) & 2u ? hi : lo;
+        }
+    } else if constexpr (FMT == kFmtTernary) {
+        // code t: 12 bits from bit 12 t, within the two bytes from 3 t / 2 (one load, no branch
+        // between even and odd codes)
+        const int64_t t = e >> 3;
+        uint16_t pair;
+        __builtin_memcpy(&pair, packed + ((3 * t) >> 1), 2);
+        uint32_t raw = 2u * (((uint32_t)pair >> (4 * (t & 1))) & 0xFFFu);
+        if (V == 4 && (e & 4)) raw = (raw * 25891u) >> 21;  // / 81, exact below 8192
+        const uint32_t vm = out_bits<ODT>(-1.0f * s), vz = out_bits<ODT>(0.0f * s),
+                       vp = out_bits<ODT>(s);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-        } else {
-            uint32_t h[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                uint32_t lo, hi;
-                if constexpr (ODT == kF16) { lo = f32_to_f16_bits(v[2 * i]); hi = f32_to_f16_bits(v[2 * i + 1]); }
-                else { lo = f32_to_bf16_bits(v[2 * i]); hi = f32_to_bf16_bits(v[2 * i + 1]); }
-                h[i] = lo | (hi << 16);
-            }
-            uint4* o = reinterpret_cast<uint4*>((uint16_t*)out + e0);
-            o[0] = make_uint4(h[0], h[1], h[2], h[3]);
-            o[1] = make_uint4(h[4], h[5], h[6], h[7]);
+        for (int i = 0; i < V; ++i) {
+            const uint32_t q = (raw * 43691u) >> 17;  // / 3, exact below 2^17
+            const uint32_t d = raw - 3u * q;
+            v[i] = d == 0u ? vm : d == 1u ? vz : vp;
+            raw = q;
         }
     } else {
+        uint32_t row[V / 4];  // the code's coordinates, one load
+        __builtin_memcpy(row, &kRootTable.c[packed[e >> 3]][e & 7], V);
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (e0 + i < numel) store_from_f32<ODT>(out, e0 + i, v[i]);
+        for (int i = 0; i < V; ++i)
+            v[i] = out_bits<ODT>((float)(int8_t)(row[i / 4] >> (8 * (i & 3))) * s);
+    }
+}
+
+// P: pieces per lane; gs_shift: log2 of the group size, or -1 where it is no power of two
+template <int FMT, int ODT, int P>
+__global__ __launch_bounds__(kDecThreads) void decode_kernel(
+    const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales, int64_t numel,
+    int64_t gs, int gs_shift, bool vec_ok, void* __restrict__ out) {
+    constexpr int V = ODT == kF32 ? 4 : 8;
+    const int64_t first = ((int64_t)blockIdx.x * (P * kDecThreads) + threadIdx.x) * V;
+    const int64_t last = (numel - 1) / V * V;  // run that pieces past the end repeat, unstored
+    uint32_t v[P][V];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int64_t e0 = first + (int64_t)p * (kDecThreads * V), e = e0 < last ? e0 : last;
+        const uint32_t s16 = scales[gs_shift >= 0 ? e >> gs_shift : e / gs];
+        decode_run<FMT, ODT, V>(packed, e, s16, v[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int64_t e = first + (int64_t)p * (kDecThreads * V);
+        if (vec_ok && e + V <= numel) {
+            if constexpr (ODT == kF32)
+                *reinterpret_cast<uint4*>((uint32_t*)out + e) =
+                    make_uint4(v[p][0], v[p][1], v[p][2], v[p][3]);
+            else
+                *reinterpret_cast<uint4*>((uint16_t*)out + e) =
+                    make_uint4(v[p][0] | (v[p][1] << 16), v[p][2] | (v[p][3] << 16),
+                               v[p][4] | (v[p][5] << 16), v[p][6] | (v[p][7] << 16));
+        } else {
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                if (e + i >= numel) continue;
+                if constexpr (ODT == kF32) ((uint32_t*)out)[e + i] = v[p][i];
+                else ((uint16_t*)out)[e + i] = (uint16_t)v[p][i];
+            }
+        }
+    }
+}
+
+// Four pieces per lane share its index work and keep four loads in flight; a tensor that
+// then leaves CUs idle takes one (512 x 512 ternary to fp16: 3.5 against 2.5 us).
+template <int FMT, int ODT>
+static hipError_t launch_decode_t(const uint8_t* packed, const uint16_t* scales, int64_t numel,
+                                  int64_t gs, void* out, hipStream_t stream) {
+    constexpr int64_t kPerBlock = kDecThreads * (ODT == kF32 ? 4 : 8);
+    const int shift = (gs & (gs - 1)) == 0 ? 63 - __builtin_clzll((unsigned long long)gs) : -1;
+    const bool vec = ((uintptr_t)out & 15u) == 0;
+    const int64_t runs = (numel + kPerBlock - 1) / kPerBlock;
+    if (runs >= 256 * kDecPieces)
+        hipLaunchKernelGGL((decode_kernel<FMT, ODT, kDecPieces>),
+                           dim3((unsigned)((runs + kDecPieces - 1) / kDecPieces)),
+                           dim3(kDecThreads), 0, stream, packed, scales, numel, gs, shift, vec, out);
+    else
+        hipLaunchKernelGGL((decode_kernel<FMT, ODT, 1>), dim3((unsigned)runs), dim3(kDecThreads), 0,
+                           stream, packed, scales, numel, gs, shift, vec, out);
+    return hipGetLastError();
+}
+
+template <int FMT>
+static hipError_t launch_decode_fmt(const uint8_t* packed, const uint16_t* scales, int64_t numel,
+                                    int64_t gs, int odt, void* out, hipStream_t stream) {
+    switch (odt) {
+        case kF32: return launch_decode_t<FMT, kF32>(packed, scales, numel, gs, out, stream);
+        case kF16: return launch_decode_t<FMT, kF16>(packed, scales, numel, gs, out, stream);
+        default: return launch_decode_t<FMT, kBF16>(packed, scales, numel, gs, out, stream);
     }
 }
 
 hipError_t launch_decode(const uint8_t* packed, const uint16_t* scales, int64_t numel, int64_t gs,
                          int odt, void* out, hipStream_t stream) {
-    const int64_t pairs = (numel + 15) / 16;
-    const int64_t blocks = (pairs + kDecThreads - 1) / kDecThreads;
-    const bool vec_ok = (((uintptr_t)out) & 15u) == 0;
-    switch (odt) {
-        case kF32:
-            hipLaunchKernelGGL((decode_kernel<kF32>), dim3((unsigned)blocks), dim3(kDecThreads), 0,
-                               stream, packed, scales, numel, gs, vec_ok, out);
-            break;
-        case kF16:
-            hipLaunchKernelGGL((decode_kernel<kF16>), dim3((unsigned)blocks), dim3(kDecThreads), 0,
-                               stream, packed, scales, numel, gs, vec_ok, out);
-            break;
-        default:
-            hipLaunchKernelGGL((decode_kernel<kBF16>), dim3((unsigned)blocks), dim3(kDecThreads), 0,
-                               stream, packed, scales, numel, gs, vec_ok, out);
-            break;
-    }
-    return hipGetLastError();
+    return launch_decode_fmt<kFmtTernary>(packed, scales, numel, gs, odt, out, stream);
+}
+
+hipError_t launch_decode2(const uint8_t* packed, const uint16_t* scales, int64_t numel,
+                          int64_t gs, int odt, void* out, hipStream_t stream) {
+    return launch_decode_fmt<kFmt2Bit>(packed, scales, numel, gs, odt, out, stream);
+}
+
+hipError_t launch_decode1(const uint8_t* codes, const uint16_t* scales, int64_t numel,
+                          int64_t gs, int odt, void* out, hipStream_t stream) {
+    return launch_decode_fmt<kFmtRoot>(codes, scales, numel, gs, odt, out, stream);
 }
 
 // ---------------------------------------------------------------- 2-bit encoder
@@ -600,79 +676,6 @@ hipError_t launch_encode2(const void* w, int wdt, int64_t numel, int64_t gs, uin
         case kF16: return launch_encode2_t<kF16>(w, numel, gs, packed, scales, stream);
         default: return launch_encode2_t<kBF16>(w, numel, gs, packed, scales, stream);
     }
-}
-
-// ---------------------------------------------------------------- 2-bit decoder
-//
-// E8LatticePacker.unpack (lattice.py:252-279): one lane per 16 weights (4 bytes), each
-// (code - 1.5) * scales.to(dtype) rounded once to dtype.
-
-template <int ODT>
-__global__ __launch_bounds__(kDecThreads) void decode2_kernel(
-    const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales, int64_t numel,
-    int64_t padded, int64_t gs, bool vec_ok, void* __restrict__ out) {
-    const int64_t p = (int64_t)blockIdx.x * kDecThreads + threadIdx.x;
-    const int64_t e0 = p * 16;
-    if (e0 >= numel) return;
-    uint32_t word;
-    if (e0 + 16 <= padded && (((uintptr_t)packed) & 3u) == 0) {
-        word = *reinterpret_cast<const uint32_t*>(packed + e0 / 4);
-    } else {
-        word = 0;
-        for (int b = 0; b < 4 && e0 + 4 * b < padded; ++b)
-            word |= (uint32_t)packed[e0 / 4 + b] << (8 * b);
-    }
-    const uint32_t s0 = scales[e0 / gs];  // gs % 8 == 0: each run of 8 is one group
-    const uint32_t s1 = (e0 + 8 < padded) ? scales[(e0 + 8) / gs] : s0;
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = deq2_value<ODT>((word >> (2 * i)) & 3u, i < 8 ? s0 : s1);
-    if (vec_ok && e0 + 16 <= numel) {
-        if constexpr (ODT == kF32) {
-            float4* o = reinterpret_cast<float4*>((float*)out + e0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-        } else {
-            uint32_t h[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                uint32_t lo, hi;
-                if constexpr (ODT == kF16) { lo = f32_to_f16_bits(v[2 * i]); hi = f32_to_f16_bits(v[2 * i + 1]); }
-                else { lo = f32_to_bf16_bits(v[2 * i]); hi = f32_to_bf16_bits(v[2 * i + 1]); }
-                h[i] = lo | (hi << 16);
-            }
-            uint4* o = reinterpret_cast<uint4*>((uint16_t*)out + e0);
-            o[0] = make_uint4(h[0], h[1], h[2], h[3]);
-            o[1] = make_uint4(h[4], h[5], h[6], h[7]);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (e0 + i < numel) store_from_f32<ODT>(out, e0 + i, v[i]);
-    }
-}
-
-hipError_t launch_decode2(const uint8_t* packed, const uint16_t* scales, int64_t numel,
-                          int64_t gs, int odt, void* out, hipStream_t stream) {
-    const int64_t padded = numel + (gs - numel % gs) % gs;
-    const int64_t quads = (numel + 15) / 16;
-    const int64_t blocks = (quads + kDecThreads - 1) / kDecThreads;
-    const bool vec_ok = (((uintptr_t)out) & 15u) == 0;
-    switch (odt) {
-        case kF32:
-            hipLaunchKernelGGL((decode2_kernel<kF32>), dim3((unsigned)blocks), dim3(kDecThreads), 0,
-                               stream, packed, scales, numel, padded, gs, vec_ok, out);
-            break;
-        case kF16:
-            hipLaunchKernelGGL((decode2_kernel<kF16>), dim3((unsigned)blocks), dim3(kDecThreads), 0,
-                               stream, packed, scales, numel, padded, gs, vec_ok, out);
-            break;
-        default:
-            hipLaunchKernelGGL((decode2_kernel<kBF16>), dim3((unsigned)blocks), dim3(kDecThreads),
-                               0, stream, packed, scales, numel, padded, gs, vec_ok, out);
-            break;
-    }
-    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- 1-bit Root-E8 encoder
@@ -867,78 +870,6 @@ hipError_t launch_encode1(const void* w, int wdt, int64_t numel, int64_t gs, uin
         case kF16: return launch_encode1_t<kF16>(w, numel, gs, codes, scales, stream);
         default: return launch_encode1_t<kBF16>(w, numel, gs, codes, scales, stream);
     }
-}
-
-// ---------------------------------------------------------------- 1-bit decoder
-//
-// RootE8LatticePacker.unpack (lattice.py:519-533): one lane per 16 weights (two codes),
-// table[code][k] * scales.to(dtype) rounded to dtype (the fp32 product is exact).
-
-template <int ODT>
-__global__ __launch_bounds__(kDecThreads) void decode1_kernel(
-    const uint8_t* __restrict__ codes, const uint16_t* __restrict__ scales, int64_t numel,
-    int64_t padded, int64_t gs, bool vec_ok, void* __restrict__ out) {
-    const int64_t p = (int64_t)blockIdx.x * kDecThreads + threadIdx.x;
-    const int64_t e0 = p * 16;
-    if (e0 >= numel) return;
-    const uint32_t c0 = codes[e0 / 8];
-    const uint32_t c1 = (e0 + 8 < padded) ? codes[e0 / 8 + 1] : 0u;
-    const uint32_t s0 = scales[e0 / gs];
-    const uint32_t s1 = (e0 + 8 < padded) ? scales[(e0 + 8) / gs] : s0;
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float q = (float)kRootTable.c[i < 8 ? c0 : c1][i & 7];
-        float prod = q * scale_for<ODT>(i < 8 ? s0 : s1);
-        keep_f32(prod);
-        v[i] = prod;
-    }
-    if (vec_ok && e0 + 16 <= numel) {
-        if constexpr (ODT == kF32) {
-            float4* o = reinterpret_cast<float4*>((float*)out + e0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-        } else {
-            uint32_t h[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                uint32_t lo, hi;
-                if constexpr (ODT == kF16) { lo = f32_to_f16_bits(v[2 * i]); hi = f32_to_f16_bits(v[2 * i + 1]); }
-                else { lo = f32_to_bf16_bits(v[2 * i]); hi = f32_to_bf16_bits(v[2 * i + 1]); }
-                h[i] = lo | (hi << 16);
-            }
-            uint4* o = reinterpret_cast<uint4*>((uint16_t*)out + e0);
-            o[0] = make_uint4(h[0], h[1], h[2], h[3]);
-            o[1] = make_uint4(h[4], h[5], h[6], h[7]);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (e0 + i < numel) store_from_f32<ODT>(out, e0 + i, v[i]);
-    }
-}
-
-hipError_t launch_decode1(const uint8_t* codes, const uint16_t* scales, int64_t numel,
-                          int64_t gs, int odt, void* out, hipStream_t stream) {
-    const int64_t padded = numel + (gs - numel % gs) % gs;
-    const int64_t pairs = (numel + 15) / 16;
-    const int64_t blocks = (pairs + kDecThreads - 1) / kDecThreads;
-    const bool vec_ok = (((uintptr_t)out) & 15u) == 0;
-    switch (odt) {
-        case kF32:
-            hipLaunchKernelGGL((decode1_kernel<kF32>), dim3((unsigned)blocks), dim3(kDecThreads), 0,
-                               stream, codes, scales, numel, padded, gs, vec_ok, out);
-            break;
-        case kF16:
-            hipLaunchKernelGGL((decode1_kernel<kF16>), dim3((unsigned)blocks), dim3(kDecThreads), 0,
-                               stream, codes, scales, numel, padded, gs, vec_ok, out);
-            break;
-        default:
-            hipLaunchKernelGGL((decode1_kernel<kBF16>), dim3((unsigned)blocks), dim3(kDecThreads),
-                               0, stream, codes, scales, numel, padded, gs, vec_ok, out);
-            break;
-    }
-    return hipGetLastError();
 }
 
 }  // namespace ojx
