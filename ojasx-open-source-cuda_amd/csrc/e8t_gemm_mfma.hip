@@ -1069,11 +1069,20 @@ static hipError_t launch_cfg(const void* x, const uint8_t* packed, const uint16_
 //  * otherwise small tiles, split over K towards two workgroups per CU (the small
 //    configuration's residency), at least kMinSplitSteps K steps per split (8: at 4 the
 //    fp32 partials of the k/v shape at M = 512 cost more than the extra workgroups gain;
-//    16 for the backward dX, whose k/v shape at M = 512 runs 12% faster unsplit).
+//    16 for the backward dX, whose k/v shape at M = 512 runs 12% faster unsplit);
+//  * one row of small tiles (M <= 128) whose grid fits twice into the CUs: split to at most
+//    one workgroup per CU, at least kMinRowSplitSteps K steps per split.  The partials of so
+//    few rows cost little, and a second workgroup on some of the CUs costs more than it
+//    hides (ternary gs 32, us from a graph, towards 512 workgroups with 8 and 16 steps
+//    against this: forward 64 rows of 1024 x 1024 15.0 and 12.3, 1024 x 4096 17.8 and 16.6;
+//    backward dX 64 rows of 1024 x 1024 22.8 and 13.6, 1024 x 4096 23.2 and 15.2, 4096 x 4096
+//    26.7 and 22.3, 17 rows of it 24.7 and 19.2; at 256 rows of 1024 x 4096 the forward
+//    loses, 20.4 and 22.8).
 // The fp32 partial sums of a split stay under kSplitBytesMax.
 constexpr int kMaxSplits = 16;
 constexpr int64_t kMinSplitSteps = 8;
 constexpr int64_t kMinSplitStepsBwd = 16;
+constexpr int64_t kMinRowSplitSteps = 4;
 constexpr int64_t kMinLargeSplitSteps = 16;
 constexpr int64_t kSplitBytesMax = 256ll << 20;
 constexpr int64_t kLargeTargetWgs = 256;
@@ -1096,6 +1105,9 @@ GemmChoice gemm_mfma_choice(int64_t M, int64_t N, int64_t K, bool bwd) {
     if (large * sl >= kLargeMinWgs) return GemmChoice{false, (int)sl};
     const int64_t tiles = ((M + CfgSmall::BM - 1) / CfgSmall::BM) *
                           ((N + CfgSmall::BN - 1) / CfgSmall::BN);
+    const int64_t fit = kLargeTargetWgs / tiles;
+    if (M <= CfgSmall::BM && fit >= 2)  // fit * tiles workgroups at most
+        return GemmChoice{true, (int)splits_for(tiles, fit * tiles, kMinRowSplitSteps, M, N, K)};
     return GemmChoice{true,
                       (int)splits_for(tiles, 512,
                                       bwd ? kMinSplitStepsBwd : kMinSplitSteps, M, N, K)};
