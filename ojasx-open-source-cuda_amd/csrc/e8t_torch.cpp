@@ -87,6 +87,21 @@ bool layer_ok(const Tensor& packed, const Tensor& scales, int fmt, int64_t N, in
            packed.numel() >= code_bytes(fmt, padded) && scales.numel() >= padded / gs;
 }
 
+// The interpreter lock is given up while memory is allocated and kernels are launched, as the
+// registered ops do: both can wait (a full queue, a new segment), and other threads go on.
+class Unlocked {
+  public:
+    Unlocked() : state_(PyEval_SaveThread()) {}
+    ~Unlocked() { lock(); }
+    void lock() {
+        if (state_) PyEval_RestoreThread(state_);
+        state_ = nullptr;
+    }
+
+  private:
+    PyThreadState* state_;
+};
+
 void* data(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 void* current_stream(const c10::Device& d) {
@@ -165,6 +180,7 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
         Py_RETURN_NONE;
     if (c10::GradMode::is_enabled() && (records(x) || records(bias))) Py_RETURN_NONE;
     RECORD_FUNCTION("ojasx_e8t::linear", std::vector<c10::IValue>());
+    Unlocked unlocked;
     const c10::DeviceGuard on_device(x.device());
     const Tensor xc = x.contiguous();
     const int64_t M = xc.numel() / K;
@@ -176,6 +192,7 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
                     data(bias), data(y), M, N, K, gs, dt, data(ws), bytes,
                     current_stream(x.device())),
           "gemm_fwd");
+    unlocked.lock();
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -194,6 +211,7 @@ PyObject* linear_bwd(PyObject*, PyObject* const* argv, Py_ssize_t n) {
         (c10::GradMode::is_enabled() && records(gy)))
         Py_RETURN_NONE;
     RECORD_FUNCTION("ojasx_e8t::linear_bwd", std::vector<c10::IValue>());
+    Unlocked unlocked;
     const c10::DeviceGuard on_device(gy.device());
     const Tensor gc = gy.contiguous();
     const int64_t M = gc.numel() / N;
@@ -204,6 +222,7 @@ PyObject* linear_bwd(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     check(kBwd[fmt](data(gc), (const uint8_t*)data(packed), (const uint16_t*)data(scales), data(gx),
                     M, N, K, gs, dt, data(ws), bytes, current_stream(gy.device())),
           "gemm_bwd_dx");
+    unlocked.lock();
     return THPVariable_Wrap(std::move(gx));
     END_HANDLE_TH_ERRORS
 }
@@ -240,6 +259,7 @@ PyObject* linear_lora(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     if (c10::GradMode::is_enabled() && (records(x) || records(bias) || records(la) || records(lb)))
         Py_RETURN_NONE;
     RECORD_FUNCTION("ojasx_e8t::linear_lora", std::vector<c10::IValue>());
+    Unlocked unlocked;
     const c10::DeviceGuard on_device(x.device());
     const Tensor xc = x.contiguous();
     const int64_t M = xc.numel() / K, r = la.size(1);
@@ -252,6 +272,7 @@ PyObject* linear_lora(PyObject*, PyObject* const* argv, Py_ssize_t n) {
                         data(bias), data(la), data(lb), r, scaling, (float*)data(u), data(y), M, N,
                         K, gs, dt, data(ws), bytes, current_stream(x.device())),
           "gemm_fwd_lora");
+    unlocked.lock();
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -278,6 +299,7 @@ PyObject* linear_lora_bwd(PyObject*, PyObject* const* argv, Py_ssize_t n) {
         x.numel() / K != gy.numel() / N || c10::GradMode::is_enabled())
         Py_RETURN_NONE;
     RECORD_FUNCTION("ojasx_e8t::linear_lora_bwd", std::vector<c10::IValue>());
+    Unlocked unlocked;
     const c10::DeviceGuard on_device(x.device());
     const Tensor xc = x.contiguous(), gc = gy.contiguous();
     const int64_t M = xc.numel() / K, r = la.size(1);
@@ -294,6 +316,7 @@ PyObject* linear_lora_bwd(PyObject*, PyObject* const* argv, Py_ssize_t n) {
                             (float*)data(uv), data(gx), data(ga), data(gb), M, N, K, gs, dt,
                             data(ws), bytes, current_stream(x.device())),
           "gemm_bwd_lora");
+    unlocked.lock();
     PyObject* out = PyTuple_New(3);
     if (!out) throw python_error();
     Tensor* ts[] = {&gx, &ga, &gb};
@@ -328,6 +351,7 @@ PyObject* encode(PyObject*, PyObject* const* argv, Py_ssize_t n) {
         (c10::GradMode::is_enabled() && records(w)))
         Py_RETURN_NONE;
     RECORD_FUNCTION("ojasx_e8t::encode", std::vector<c10::IValue>());
+    Unlocked unlocked;
     const c10::DeviceGuard on_device(w.device());
     const Tensor wc = w.contiguous();
     const int64_t padded = padded_to(wc.numel(), gs);
@@ -336,6 +360,7 @@ PyObject* encode(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     check(kEncode[fmt](data(wc), dt, wc.numel(), gs, (uint8_t*)data(packed),
                        (uint16_t*)data(scales), current_stream(w.device())),
           "encode");
+    unlocked.lock();
     PyObject* out = PyTuple_New(2);
     if (!out) throw python_error();
     PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(packed)));
@@ -362,12 +387,14 @@ PyObject* decode(PyObject*, PyObject* const* argv, Py_ssize_t n) {
         (c10::GradMode::is_enabled() && records(scales)))
         Py_RETURN_NONE;
     RECORD_FUNCTION("ojasx_e8t::decode", std::vector<c10::IValue>());
+    Unlocked unlocked;
     const c10::DeviceGuard on_device(packed.device());
     const at::ScalarType types[] = {at::kFloat, at::kHalf, at::kBFloat16};
     Tensor out = at::empty({numel}, packed.options().dtype(types[dt]));
     check(kDecode[fmt]((const uint8_t*)data(packed), (const uint16_t*)data(scales), numel, gs, dt,
                        data(out), current_stream(packed.device())),
           "decode");
+    unlocked.lock();
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
