@@ -275,6 +275,18 @@ def _check_fmt_layer(fmt: int, packed_weight: torch.Tensor, block_scales: torch.
         raise RuntimeError(f"unknown weight format {fmt}")
 
 
+def _check_factors(lora_a: torch.Tensor, lora_b: torch.Tensor, out_features: int,
+                   in_features: int) -> int:
+    """The adapter's rank; its factors must be [in, r] and [r, out]."""
+    r = lora_a.shape[-1]
+    if lora_a.dim() != 2 or lora_a.shape[0] != in_features or tuple(lora_b.shape) != (r, out_features):
+        raise RuntimeError(f"LoRA factors must be [{in_features}, r] and [r, {out_features}] "
+                           f"(got {tuple(lora_a.shape)} and {tuple(lora_b.shape)})")
+    if not 1 <= r <= LORA_MAX_RANK:
+        raise RuntimeError(f"fused LoRA supports ranks 1..{LORA_MAX_RANK} (got {r})")
+    return r
+
+
 @torch.library.custom_op(f"{_NS}::linear_lora", mutates_args=())
 def linear_lora(x: torch.Tensor, packed_weight: torch.Tensor, block_scales: torch.Tensor,
                 bias: Optional[torch.Tensor], lora_a: torch.Tensor, lora_b: torch.Tensor,
@@ -287,12 +299,7 @@ def linear_lora(x: torch.Tensor, packed_weight: torch.Tensor, block_scales: torc
     if x.shape[-1] != in_features:
         raise RuntimeError(f"x has {x.shape[-1]} features, layer expects {in_features}")
     _check_fmt_layer(fmt, packed_weight, block_scales, out_features, in_features, group_size)
-    r = lora_a.shape[-1]
-    if lora_a.dim() != 2 or lora_a.shape[0] != in_features or tuple(lora_b.shape) != (r, out_features):
-        raise RuntimeError(f"LoRA factors must be [{in_features}, r] and [r, {out_features}] "
-                           f"(got {tuple(lora_a.shape)} and {tuple(lora_b.shape)})")
-    if not 1 <= r <= LORA_MAX_RANK:
-        raise RuntimeError(f"fused LoRA supports ranks 1..{LORA_MAX_RANK} (got {r})")
+    r = _check_factors(lora_a, lora_b, out_features, in_features)
     dt = _dtype_code(x.dtype)
     x2 = x.reshape(-1, in_features).contiguous()
     M = x2.shape[0]
@@ -347,6 +354,19 @@ def linear_lora_bwd(x: torch.Tensor, grad_y: torch.Tensor, packed_weight: torch.
     epilogue.  Every operand in grad_y's dtype, at least one row."""
     dev = N.require_device(x, grad_y, packed_weight, block_scales, lora_a, lora_b)
     dt = _dtype_code(grad_y.dtype)
+    # the kernels take every size from grad_y and the integers
+    if x.dim() < 1 or x.shape[-1] != in_features:
+        raise RuntimeError(f"x is {tuple(x.shape)}, layer expects {in_features} features")
+    if grad_y.dim() < 1 or grad_y.shape[-1] != out_features:
+        raise RuntimeError(f"grad_y is {tuple(grad_y.shape)}, expected {out_features} features")
+    _check_fmt_layer(fmt, packed_weight, block_scales, out_features, in_features, group_size)
+    _check_factors(lora_a, lora_b, out_features, in_features)
+    for what, t in (("x", x), ("lora_a", lora_a), ("lora_b", lora_b)):
+        if t.dtype != grad_y.dtype:
+            raise RuntimeError(f"{what} is {t.dtype}, grad_y {grad_y.dtype}")
+    if grad_y.numel() == 0 or x.numel() * out_features != grad_y.numel() * in_features:
+        raise RuntimeError(f"x {tuple(x.shape)} and grad_y {tuple(grad_y.shape)} must have the "
+                           "same number of rows, at least one")
     x2 = x.reshape(-1, in_features).contiguous()
     gy = grad_y.reshape(-1, out_features).contiguous()
     la, lb = lora_a.contiguous(), lora_b.contiguous()
