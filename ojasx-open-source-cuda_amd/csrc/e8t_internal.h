@@ -229,7 +229,9 @@ hipError_t launch_lora_down(const void* x, int64_t M, int64_t K, int dt, const L
 // (x @ A) and v = scaling * (gy @ B^T), fp32 [M, r] each.
 //   launch_lora_uv: u and / or v (either null to skip it), one launch;
 //   launch_lora_grads: grad_a and / or grad_b in dtype; row splits of the sums over M leave
-//   fp32 partials, lora_grads_bytes in all, in `part` (smaller or null: one split).
+//   fp32 partials, lora_grads_bytes in all, in `part` (smaller: fewer splits; null: one).
+// Any M; N and K under kLoraGradMaxWidth (32-bit buffer offsets over a few rows).
+constexpr int64_t kLoraGradMaxWidth = 1ll << 23;
 hipError_t launch_lora_uv(const void* x, const void* gy, const void* a, const void* b,
                           float scaling, int64_t M, int64_t N, int64_t K, int64_t r, int dt,
                           float* u, float* v, hipStream_t stream);

@@ -500,11 +500,14 @@ struct LoraGradArgs {
     float* part;     // fp32 partial sums of the row splits (gridDim.y > 1)
     int64_t M, total;  // total: values per split
     int r, blocks0;  // blocks0: workgroups of it[0]
+    int span;        // groups of four rows per buffer
 };
 
 // A wave owns 128 columns c: lane (g, i) loads a[m0 + g][8 i .. 8 i + 7], eight instructions
 // of four rows each (instruction e: columns 8 i + e).  The workgroup's waves and gridDim.y
 // split the rows.  VEC: rows of a hold whole aligned groups of eight.
+// A wave walks its rows through buffers of args.span groups (offsets are 32 bits wide), so
+// any M runs with any number of row splits.
 constexpr int kLoraGradWaves = 8;
 
 template <int DT, int NT, bool VEC>
@@ -524,26 +527,19 @@ __global__ __launch_bounds__(64 * kLoraGradWaves) void lora_grad_kernel(LoraGrad
     const int64_t parts = (int64_t)gridDim.y * kLoraGradWaves;
     const int64_t p = (int64_t)blockIdx.y * kLoraGradWaves + wave;
     const int64_t q_begin = groups * p / parts;
-    const int count = (int)(groups * (p + 1) / parts - q_begin);
+    const int64_t count = groups * (p + 1) / parts - q_begin;
     const int64_t m_begin = 4 * q_begin;
-    // the wave's rows; the rows past its last belong to others or lie past the end
-    const int64_t left = args.M - m_begin < 4 * count ? args.M - m_begin : 4 * count;
-    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(static_cast<const char*>(it.a) + m_begin * it.C * E), (short)0,
-        (int)(left * it.C * E), kRsrcWord3);
-    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(it.v + m_begin * r), (short)0, (int)(left * r * 4), kRsrcWord3);
-
     struct Batch {
         RawX<DT, 8> a[U];
         uint32_t v[U][NT];
     };
-    auto load = [&](Batch& f, int q) {
+    // groups q .. q + U - 1 of a buffer of n groups
+    auto load = [&](Batch& f, __amdgpu_buffer_rsrc_t ar, __amdgpu_buffer_rsrc_t vr, int n, int q) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t m = 4 * (uint32_t)(q + u) + g;
             const uint32_t base = m * (uint32_t)it.C + (uint32_t)c0;
-            const bool live = q + u < count;
+            const bool live = q + u < n;
             if constexpr (VEC) {
                 f.a[u].load(ar, live && c0 < it.C ? base * E : kNoRecordOffset);
             } else {
@@ -580,15 +576,26 @@ __global__ __launch_bounds__(64 * kLoraGradWaves) void lora_grad_kernel(LoraGrad
                 for (int t = 0; t < NT; ++t)
                     acc[e][t] = mfma4(f.a[u].get(e), __uint_as_float(f.v[u][t]), acc[e][t]);
     };
-    Batch f0, f1;
-    load(f0, 0);
-    for (int q = 0; q < count; q += 2 * U) {
-        load(f1, q + U);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(f0);
-        load(f0, q + 2 * U);
-        __builtin_amdgcn_sched_barrier(0);
-        if (q + U < count) compute(f1);
+    for (int64_t q0 = 0; q0 < count; q0 += args.span) {
+        // rows past the buffer's last belong to others or lie past the end
+        const int n = (int)(count - q0 < args.span ? count - q0 : args.span);
+        const int64_t m0 = m_begin + 4 * q0;
+        const int64_t left = args.M - m0 < 4 * n ? args.M - m0 : 4 * n;
+        const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(static_cast<const char*>(it.a) + m0 * it.C * E), (short)0,
+            (int)(left * it.C * E), kRsrcWord3);
+        const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(it.v + m0 * r), (short)0, (int)(left * r * 4), kRsrcWord3);
+        Batch f0, f1;
+        load(f0, ar, vr, n, 0);
+        for (int q = 0; q < n; q += 2 * U) {
+            load(f1, ar, vr, n, q + U);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(f0);
+            load(f0, ar, vr, n, q + 2 * U);
+            __builtin_amdgcn_sched_barrier(0);
+            if (q + U < n) compute(f1);
+        }
     }
 #pragma unroll
     for (int h = kLoraGradWaves / 2; h >= 1; h /= 2) {
@@ -636,16 +643,20 @@ __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(LoraGradArgs args
     store_from_f32<DT>(it.out, i - it.at, v);
 }
 
-// Row splits: towards four waves per SIMD over the chip, at least 32 rows per wave, and the
-// rows of a wave within 32-bit buffer offsets.
-static int64_t lora_grad_splits(int64_t M, int64_t blocks, int64_t cmax) {
+// Row splits: towards four waves per SIMD over the chip, at least 32 rows per wave.
+static int64_t lora_grad_splits(int64_t M, int64_t blocks) {
     int64_t s = 4096 / (blocks * kLoraGradWaves);
     const int64_t most = M / (32 * kLoraGradWaves);
     if (s > most) s = most;
     if (s > 16) s = 16;
-    const int64_t least = M * cmax * 4 / kLoraGradWaves / (1ll << 30);
-    if (s < least) s = least;
     return s < 1 ? 1 : s;
+}
+
+// Groups of four rows per buffer: 256 MB of fp32 rows (refilling the pipeline that often costs
+// nothing), at least one trip of the loop, which at widths under kLoraGradMaxWidth is 1 GB.
+static int lora_grad_span(int64_t cmax) {
+    const int64_t n = (1ll << 28) / (cmax * 16) / 8 * 8;
+    return n < 8 ? 8 : (int)n;
 }
 
 static int64_t lora_blocks(int64_t C) { return (C + 127) / 128; }
@@ -653,7 +664,7 @@ static int64_t lora_blocks(int64_t C) { return (C + 127) / 128; }
 size_t lora_grads_bytes(int64_t M, int64_t N, int64_t K, int64_t r, bool need_a, bool need_b) {
     const int64_t blocks = (need_a ? lora_blocks(K) : 0) + (need_b ? lora_blocks(N) : 0);
     if (blocks == 0 || M < 1) return 0;
-    const int64_t s = lora_grad_splits(M, blocks, K > N ? K : N);
+    const int64_t s = lora_grad_splits(M, blocks);
     return s > 1 ? (size_t)s * (size_t)((need_a ? K : 0) + (need_b ? N : 0)) * (size_t)r * 4 : 0;
 }
 
@@ -681,7 +692,8 @@ static hipError_t launch_lora_grads_dt(const LoraGradArgs& args, int64_t blocks,
 hipError_t launch_lora_grads(const void* x, const void* gy, const float* u, const float* v,
                              int64_t M, int64_t N, int64_t K, int64_t r, int dt, void* grad_a,
                              void* grad_b, float* part, size_t part_bytes, hipStream_t stream) {
-    if (M < 1 || r < 1 || r > kLoraMaxRank) return hipErrorInvalidValue;
+    if (M < 1 || r < 1 || r > kLoraMaxRank || K >= kLoraGradMaxWidth || N >= kLoraGradMaxWidth)
+        return hipErrorInvalidValue;
     const LoraGrad ga{x, v, grad_a, K, r, 1, 0}, gb{gy, u, grad_b, N, 1, N, grad_a ? K * r : 0};
     LoraGradArgs args{};
     int n = 0;
@@ -699,12 +711,11 @@ hipError_t launch_lora_grads(const void* x, const void* gy, const float* u, cons
     args.part = part;
     args.M = M;
     args.r = (int)r;
-    int64_t splits = lora_grad_splits(M, blocks, K > N ? K : N);
+    const int64_t cmax = K > N ? K : N;
+    args.span = lora_grad_span(cmax > kLoraMaxRank ? cmax : kLoraMaxRank);
+    int64_t splits = lora_grad_splits(M, blocks);
     const int64_t fit = part ? (int64_t)(part_bytes / ((size_t)args.total * 4)) : 0;
     if (splits > fit) splits = fit < 2 ? 1 : fit;
-    if ((M / (splits * kLoraGradWaves) + 8) * (K > N ? K : N) * 4 >= (1ll << 31) ||
-        blocks > 0x7FFFFFFF)
-        return hipErrorInvalidValue;
     const int64_t n0 = args.it[0].C * r;
     return dt == kF32   ? launch_lora_grads_dt<kF32>(args, blocks, splits, vec, n0, stream)
            : dt == kF16 ? launch_lora_grads_dt<kF16>(args, blocks, splits, vec, n0, stream)
