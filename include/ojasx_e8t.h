@@ -161,8 +161,9 @@ int ojx_e8t_gemm_bwd_dx(const void* grad_y, const uint8_t* packed, const uint16_
  * lattice.py:827-846), fmt an OJX_FMT_* code: grad_x[M,K] = grad_y . Wdeq + v @ A^T, grad_a[K,rank]
  * = x^T v and grad_b[rank,N] = u^T grad_y in dtype, with u = scaling * (x @ A) and v = scaling *
  * (grad_y @ B^T) kept in fp32 in the caller's scratch lora_uv [2, M, rank].  Any of the three
- * results may be null.  M, N, K >= 1.  The workspace (ojx_gemm_bwd_lora_workspace_bytes) holds
- * the fp32 partial sums of row splits; a smaller one lowers the split counts. */
+ * results may be null.  M, N, K >= 1; N, K < 2^23 (else OJX_ELAYOUT, before any launch).  The
+ * workspace (ojx_gemm_bwd_lora_workspace_bytes) holds the fp32 partial sums of row splits; a
+ * smaller one lowers the split counts. */
 int ojx_gemm_bwd_lora(int fmt, const void* x, const void* grad_y, const uint8_t* packed,
                       const uint16_t* scales, const void* lora_a, const void* lora_b,
                       int64_t rank, float scaling, float* lora_uv, void* grad_x, void* grad_a,

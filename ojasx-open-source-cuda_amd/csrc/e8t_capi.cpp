@@ -319,6 +319,13 @@ static int gemm_bwd(int fmt, const void* grad_y, const uint8_t* packed, const ui
     return OJX_OK;
 }
 
+static int check_lora_grad_width(int64_t N, int64_t K) {
+    if (N >= ojx::kLoraGradMaxWidth || K >= ojx::kLoraGradMaxWidth)
+        return fail(OJX_ELAYOUT, "adapter gradients need N, K < %lld (N=%lld K=%lld)",
+                    (long long)ojx::kLoraGradMaxWidth, (long long)N, (long long)K);
+    return OJX_OK;
+}
+
 // Backward of a linear with a LoRA adapter, after gemm_fwd_lora's forward: v = scaling *
 // (gy @ B^T) and u = scaling * (x @ A) in fp32 (one launch), grad_x = gy . W + v @ A^T (the
 // adapter term in the backward GEMM's epilogue), grad_a = x^T v, grad_b = u^T gy.
@@ -335,6 +342,7 @@ static int gemm_bwd_lora(int fmt, const void* x, const void* grad_y, const uint8
     if (M < 1 || N < 1 || K < 1)
         return fail(OJX_EINVAL, "adapter gradients need M, N, K >= 1 (M=%lld N=%lld K=%lld)",
                     (long long)M, (long long)N, (long long)K);
+    if (int r = check_lora_grad_width(N, K)) return r;
     if (!x || !grad_y || !packed || !scales || !lora_a || !lora_b || !lora_uv)
         return fail(OJX_EINVAL, "null input pointer");
     if (((uintptr_t)lora_uv & 3u) || ((uintptr_t)lora_a & 1u) || ((uintptr_t)lora_b & 1u))
@@ -866,6 +874,7 @@ __attribute__((visibility("default"))) int ojx_gemm_bwd_lora_workspace_bytes(
     if (rank < 1 || rank > ojx::kLoraMaxRank)
         return fail(OJX_ELAYOUT, "LoRA rank must be in 1..%lld (got %lld)",
                     (long long)ojx::kLoraMaxRank, (long long)rank);
+    if (int r = check_lora_grad_width(N, K)) return r;
     if (int r = workspace_bytes(fmt, 1, M, N, K, gs, dtype, bytes)) return r;
     if (!need_x) *bytes = 0;
     const size_t g = ojx::lora_grads_bytes(M, N, K, rank, need_a != 0, need_b != 0);

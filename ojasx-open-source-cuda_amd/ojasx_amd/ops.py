@@ -258,6 +258,7 @@ e8t_linear.register_autograd(_linear_backward, setup_context=_linear_setup_conte
 _FWD_LORA = {FMT_TERNARY: "ojx_e8t_gemm_fwd_lora", FMT_E8: "ojx_e8_gemm_fwd_lora",
              FMT_ROOT: "ojx_e8r_gemm_fwd_lora"}
 LORA_MAX_RANK = 64  # ojx_lora_down's rank range (include/ojasx_e8t.h)
+LORA_BWD_WIDTH_END = 1 << 23  # ojx_gemm_bwd_lora takes narrower layers
 
 
 def _check_fmt_layer(fmt: int, packed_weight: torch.Tensor, block_scales: torch.Tensor,
@@ -403,7 +404,8 @@ def _(x, grad_y, packed_weight, block_scales, lora_a, lora_b, scaling, fmt, out_
 def _linear_lora_backward(ctx, grad_y):
     """grad_x through the fused backward dX plus the adapter's term, and the adapter's own
     gradients: one fused op, or torch products where the gradients themselves are to be
-    differentiated (create_graph) or there are no rows; the bias's gradient in torch."""
+    differentiated (create_graph), there are no rows or the layer is too wide; the bias's
+    gradient in torch."""
     x, packed_weight, block_scales, lora_a, lora_b = ctx.saved_tensors
     out_features, in_features, group_size = ctx.dims
     sc = ctx.scaling
@@ -413,7 +415,8 @@ def _linear_lora_backward(ctx, grad_y):
     grad_x = grad_a = grad_b = grad_bias = None
     if ctx.has_bias and ctx.needs_input_grad[3]:
         grad_bias = grad_y.reshape(-1, out_features).sum(dim=0).to(ctx.bias_dtype)
-    if not torch.is_grad_enabled() and grad_y.numel() > 0 and x.dtype == grad_y.dtype:
+    if (not torch.is_grad_enabled() and grad_y.numel() > 0 and x.dtype == grad_y.dtype
+            and max(out_features, in_features) < LORA_BWD_WIDTH_END):
         if need_x or need_a or need_b:
             out = None
             if not torch.compiler.is_compiling():
