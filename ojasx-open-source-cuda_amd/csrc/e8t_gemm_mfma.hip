@@ -1097,14 +1097,8 @@ static hipError_t launch_cfg(const void* x, const uint8_t* packed, const uint16_
 //    configuration's residency), at least kMinSplitSteps K steps per split (8: at 4 the
 //    fp32 partials of the k/v shape at M = 512 cost more than the extra workgroups gain;
 //    16 for the backward dX, whose k/v shape at M = 512 runs 12% faster unsplit);
-//  * one row of small tiles (M <= 128) whose grid fits twice into the CUs: split to at most
-//    one workgroup per CU, at least kMinRowSplitSteps K steps per split.  The partials of so
-//    few rows cost little, and a second workgroup on some of the CUs costs more than it
-//    hides (ternary gs 32, us from a graph, towards 512 workgroups with 8 and 16 steps
-//    against this: forward 64 rows of 1024 x 1024 15.0 and 12.3, 1024 x 4096 17.8 and 16.6;
-//    backward dX 64 rows of 1024 x 1024 22.8 and 13.6, 1024 x 4096 23.2 and 15.2, 4096 x 4096
-//    26.7 and 22.3, 17 rows of it 24.7 and 19.2; at 256 rows of 1024 x 4096 the forward
-//    loses, 20.4 and 22.8).
+//  * one row of at most 128 small tiles (M <= 128): the split that row_split_cost puts
+//    lowest.
 // The fp32 partial sums of a split stay under kSplitBytesMax.
 constexpr int kMaxSplits = 16;
 constexpr int64_t kMinSplitSteps = 8;
@@ -1124,6 +1118,32 @@ static int64_t splits_for(int64_t tiles, int64_t target, int64_t min_steps, int6
     return s < 1 ? 1 : s;
 }
 
+// Time of a split of one row of tiles, in 0.1 us and up to a constant: the K steps of a
+// workgroup, slower where CUs hold two of them, and the fp32 partials, which cost a second
+// launch and their writes and reads (partly behind the other workgroup's steps).  Fitted to the
+// times of ternary gs 32 layers in bf16 (256 to 14336 columns out of 512 to 14336, M = 1 to 128,
+// forward and backward dX, us from a graph), where its choice is 0.2% from the best on
+// average (0.1% over 500 random layers of every format, group size and 16-bit type).  us at 64
+// rows: forward 1024 -> 1024 in 2 splits of 8 steps 15.0, in 4 of 4 11.9; 4096 -> 8192 with one
+// workgroup per CU (4 splits) 23.3, with two 20.7; 4096 -> 11008 38.4 and (5 splits) 28.4, but 6
+// splits, four workgroups more than fit, 38.7; backward dX of 11008 columns out of 4096 42.4 and
+// 32.6.
+static int64_t row_split_cost(int64_t tiles, int64_t s, int64_t M, int64_t N, int64_t K) {
+    const bool two = tiles * s > 256;
+    const int64_t steps = (K / kBK + s - 1) / s;
+    if (s == 1) return steps * (two ? 12 : 9) + (two ? 20 : 0);
+    const int64_t kb = s * M * N * 4 / 1024;  // of partials
+    return steps * (two ? 12 : 9) + (two ? 20 : 0) + 13 + kb * (two ? 33 : 50) / 10240;
+}
+
+// At most two workgroups per CU and at least kMinRowSplitSteps K steps each.
+static int row_splits(int64_t tiles, int64_t M, int64_t N, int64_t K) {
+    int64_t best = 1;
+    for (int64_t s = 2; s <= kMaxSplits && tiles * s <= 512 && K / kBK / s >= kMinRowSplitSteps; ++s)
+        if (row_split_cost(tiles, s, M, N, K) < row_split_cost(tiles, best, M, N, K)) best = s;
+    return (int)best;
+}
+
 GemmChoice gemm_mfma_choice(int64_t M, int64_t N, int64_t K, bool bwd) {
     const int64_t large = ((M + CfgLarge::BM - 1) / CfgLarge::BM) *
                           ((N + CfgLarge::BN - 1) / CfgLarge::BN);
@@ -1132,9 +1152,7 @@ GemmChoice gemm_mfma_choice(int64_t M, int64_t N, int64_t K, bool bwd) {
     if (large * sl >= kLargeMinWgs) return GemmChoice{false, (int)sl};
     const int64_t tiles = ((M + CfgSmall::BM - 1) / CfgSmall::BM) *
                           ((N + CfgSmall::BN - 1) / CfgSmall::BN);
-    const int64_t fit = kLargeTargetWgs / tiles;
-    if (M <= CfgSmall::BM && fit >= 2)  // fit * tiles workgroups at most
-        return GemmChoice{true, (int)splits_for(tiles, fit * tiles, kMinRowSplitSteps, M, N, K)};
+    if (M <= CfgSmall::BM && tiles <= 128) return GemmChoice{true, row_splits(tiles, M, N, K)};
     return GemmChoice{true,
                       (int)splits_for(tiles, 512,
                                       bwd ? kMinSplitStepsBwd : kMinSplitSteps, M, N, K)};
