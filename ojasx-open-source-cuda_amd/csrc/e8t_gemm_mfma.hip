@@ -936,6 +936,10 @@ __global__ __launch_bounds__(C::THREADS) void gemm_mfma_kernel(
     }
 
     // ---- epilogue: lane (g, i16) holds rows 4g+q of column i16 of each 16x16 tile
+    // Ternary backward: the code loads past the last step land first.  A wait that the compiler
+    // places for one of them inside a store's row check is repeated in each of the 64 checks,
+    // and then every store waits for the one before (fp16, 256 x 64 -> 128: 13.0 us, not 8.0).
+    if constexpr (BWD && kTernary) vm_wait_le<0>();
     if (lora.r > 0)
         lora_add<DT, kTM, kTN>(acc, lora, m0 + arow0, M, NO, lane,
                                [&](int j) { return n0 + brow0 + 16 * j + i16; }, split, splits);

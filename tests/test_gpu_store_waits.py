@@ -1,0 +1,48 @@
+"""The backward dX's result stores do not wait for each other in any 16-bit type.
+
+The two types run the same instructions apart from their conversions, so their times on one
+card agree; with a wait in each store's row check one of them took 1.6 times the other's.
+"""
+
+import pytest
+import torch
+
+from ojasx_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+
+def _us(fn, launches=16):
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        for _ in range(launches):
+            fn()
+    best = float("inf")
+    for _ in range(10):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / launches)
+    return best
+
+
+@pytest.mark.parametrize("bwd,code_bytes", [
+    (ops.e8t_linear_bwd_dx, 3 / 16), (ops.e8_linear_bwd_dx, 1 / 4), (ops.e8r_linear_bwd_dx, 1 / 8)])
+@pytest.mark.parametrize("gs", [16, 32, 64])
+def test_types_agree(bwd, code_bytes, gs):
+    M, N, K = 4096, 64, 64
+    packed = torch.zeros(int(N * K * code_bytes), dtype=torch.uint8, device=DEV)
+    scales = torch.ones(N * K // gs, dtype=torch.float16, device=DEV)
+    us = [_us(lambda: bwd(gy, packed, scales, N, K, gs))
+          for gy in (torch.zeros(M, N, dtype=t, device=DEV) for t in (torch.bfloat16, torch.float16))]
+    print(f"bwd gs={gs} {us}", flush=True)
+    assert max(us) < 1.3 * min(us)
