@@ -791,8 +791,11 @@ __device__ __forceinline__ void vm_wait_le() {
 
 // FMT: kFmtTernary (group size GS2 = 16, 32 or 64), kFmt2Bit or kFmtRoot (GS2 = 8 .. 64).  BWD = false:
 // y[M, N] = x[M, K] . W[N, K]^T + bias; BWD = true: y[M, K] = x[M, N] . W[N, K] (backward
-// dX; x is grad_y, bias unused).  The weight matrix is W[N, K] in both.
-template <int DT, typename C, int FMT, int GS2, bool BWD>
+// dX; x is grad_y, bias unused).  The weight matrix is W[N, K] in both.  LORA: lora may hold an
+// adapter.  The backward of the low-bit formats on large tiles has a kernel without: the
+// adapter's code costs its main loop 3 to 4% through the register allocation (bf16, M = 4096
+// of 8192 x 4160, 2 bits gs 32 445 against 475 us); elsewhere one kernel is as fast or faster.
+template <int DT, typename C, int FMT, int GS2, bool BWD, bool LORA>
 __global__ __launch_bounds__(C::THREADS) void gemm_mfma_kernel(
     const void* __restrict__ x, const uint8_t* __restrict__ packed,
     const uint16_t* __restrict__ scales, const void* __restrict__ bias, void* __restrict__ y,
@@ -940,7 +943,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_mfma_kernel(
     // places for one of them inside a store's row check is repeated in each of the 64 checks,
     // and then every store waits for the one before (fp16, 256 x 64 -> 128: 13.0 us, not 8.0).
     if constexpr (BWD && kTernary) vm_wait_le<0>();
-    if (lora.r > 0)
+    if (LORA && lora.r > 0)
         lora_add<DT, kTM, kTN>(acc, lora, m0 + arow0, M, NO, lane,
                                [&](int j) { return n0 + brow0 + 16 * j + i16; }, split, splits);
     if (splits > 1) {  // fp32 partial sums of this K range: part[split][row][col]
@@ -1084,9 +1087,18 @@ static hipError_t launch_cfg(const void* x, const uint8_t* packed, const uint16_
     const int64_t NO = BWD ? K : N;
     const int64_t tiles = ((M + C::BM - 1) / C::BM) * ((NO + C::BN - 1) / C::BN);
     if (tiles * splits > 0x7FFFFFFF) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_mfma_kernel<DT, C, FMT, GS2, BWD>), dim3((unsigned)(tiles * splits)),
-                       dim3(C::THREADS), 0, stream, x, packed, scales, bias, y, part, splits, M,
-                       N, K, lora);
+    const dim3 grid((unsigned)(tiles * splits)), block(C::THREADS);
+    if constexpr (BWD && FMT != kFmtTernary && std::is_same_v<C, CfgLarge>) {
+        if (lora.r > 0)
+            hipLaunchKernelGGL((gemm_mfma_kernel<DT, C, FMT, GS2, BWD, true>), grid, block, 0,
+                               stream, x, packed, scales, bias, y, part, splits, M, N, K, lora);
+        else
+            hipLaunchKernelGGL((gemm_mfma_kernel<DT, C, FMT, GS2, BWD, false>), grid, block, 0,
+                               stream, x, packed, scales, bias, y, part, splits, M, N, K, lora);
+    } else {
+        hipLaunchKernelGGL((gemm_mfma_kernel<DT, C, FMT, GS2, BWD, true>), grid, block, 0, stream,
+                           x, packed, scales, bias, y, part, splits, M, N, K, lora);
+    }
     const hipError_t e = hipGetLastError();
     if (splits == 1 || e != hipSuccess) return e;
     return launch_split_reduce(part, splits, BWD ? nullptr : bias, y, M, NO, DT, stream);
