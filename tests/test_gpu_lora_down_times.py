@@ -1,0 +1,54 @@
+"""Times of the adapter's down-projection against each other on one card: pairs of calls of
+nearly the same work, one of which once took a form that did not fit it."""
+
+import pytest
+import torch
+
+from ojasx_amd import _native as N
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+f32, f16, bf16 = torch.float32, torch.float16, torch.bfloat16
+
+
+def _graph(M, K, rank, dtype, launches=12):
+    x = torch.zeros(M, K, dtype=dtype, device=DEV)
+    a = torch.zeros(K, rank, dtype=dtype, device=DEV)
+    u = torch.empty(M, rank, device=DEV)
+
+    def down():
+        N.check(N.lib().ojx_lora_down(N.ptr(x), N.ptr(a), M, K, rank, 1.0, N.DTYPE_CODE[dtype],
+                                      N.ptr(u), N.stream_handle(DEV)), "lora_down")
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        down()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        for _ in range(launches):
+            down()
+    return graph, (x, a, u)
+
+
+def _ratio(first, second):
+    """Time of the first call over the second's: the best of ten runs each, in turn."""
+    graphs = [_graph(*first), _graph(*second)]
+    best = [float("inf")] * 2
+    for _ in range(10):
+        for i, (graph, _) in enumerate(graphs):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], a.elapsed_time(b))
+    print(f"lora down {first} / {second}: {best[0] / best[1]:.2f}", flush=True)
+    return best[0] / best[1]
+
+
+@pytest.mark.parametrize("rank", [16, 24, 64])
+def test_two_workgroups_per_cu_in_both_types(rank):
+    assert _ratio((384, 4096, rank, bf16), (384, 4096, rank, f16)) < 1.12  # 1.2 with one
