@@ -463,18 +463,47 @@ static bool lora_row_ok(const LoraMul& it) {
 }
 static int lora_slices(int64_t r) { return r <= 8 ? 1 : r <= 16 ? 2 : r <= 32 ? 4 : 8; }
 
-// Rows from which the tiles of 16 rows are the faster form.  Below, a workgroup per row
-// reads the factor from L2 once per row but has its whole K in flight at once (bf16, rank 8,
-// K = 4096, rows against tiles: 64 rows 4.7 and 7.2 us, 512 6.9 and 7.4, 2048 19.6 and 8.0; fp32
-// 64 rows 6.3 and 12.1, 512 11.8 and 12.4, 2048 38.9 and 13.3; rank 64 in bf16 gains at 512:
-// 15.6 and 13.5).
-constexpr int64_t kLoraTilesFrom = 512;
+// Workgroups of the row form (one per row and product) up to which it runs: two per CU, all at
+// once.  It reads the factor from L2 once per row but has its whole K in flight; tiles of 16 rows
+// read it once per tile (us at K = 4096, rows against tiles: bf16 rank 8 512 rows 7.1 and 7.8, 640
+// rows 9.1 and 7.8; rank 64 12.9 and 13.7, 17.5 and 13.7; fp32 rank 8 12.1 and 12.6, 15.9 and
+// 12.6).
+constexpr int64_t kLoraRowForm = 512;
 // Rows below which a factor that cannot be read in 16-byte pieces takes the general kernel.
 constexpr int64_t kLoraGeneralBelow = 16;
 
+// Whether the general kernel (a workgroup per row, value by value) is faster than tiles for x @ A:
+// few ranks, and rows or factors that the tiles can only read value by value too.  Times in us
+// fitted to ranks 1 to 33, 16 to 4096 rows and K = 256 to 14336; its choice is 0.5% from the
+// faster form on average.  In us, general against tiles, 64 rows: fp32 rank 3, K = 4096 7.3 and
+// 12.0, rank 12 17.6 and 12.0; bf16 rank 3, K = 256 3.1 and 4.0, K = 4096 8.3 and 7.3; bf16 rank 8,
+// K = 1001 5.3 and 17.
+static bool lora_general_faster(const LoraMul& it, int64_t M, int dt) {
+    const bool half = dt != kF32;
+    const bool vec = it.K % 8 == 0 && (((uintptr_t)it.x | (uintptr_t)it.f) & 15u) == 0;
+    const double r = (double)it.r, k = it.K / 1024.0;
+    if (it.r > (vec ? 16 : 32)) return false;
+    // a workgroup's sums across its lanes, for as many ranks as its kernel has; and rows past one
+    // workgroup per CU: their reads of A overlap, less so where its rows share the same channels
+    const double sums = it.r <= 8 ? 3.0 : it.r <= 16 ? 3.6 : 5.2;
+    const double more_sums = it.r <= 8 ? 0.45 : it.r <= 16 ? 1.1 : 2.2;
+    const double rows = M > 256 ? M / 256.0 - 1.0 : 0.0;
+    const double share = it.r % 8 == 0 ? 0.8 : it.r < 8 ? (half ? 0.3 : 0.35) : (half ? 0.4 : 0.6);
+    const double per_k = (half ? 0.7 + 0.24 * r : 0.4 + 0.25 * r) * (it.r % 16 == 0 ? 1.7 : 1.0);
+    const double general = sums + more_sums * rows + k * (1.0 + share * rows) * per_k;
+    double tiles;
+    if (half) {
+        tiles = !vec ? 10.0 + k * (it.r > 16 ? 4.5 : 7.0)
+                     : 5.0 + 0.55 * k > 2.8 + 1.14 * k ? 5.0 + 0.55 * k : 2.8 + 1.14 * k;
+    } else {
+        tiles = vec ? 4.8 + 2.0 * k : 6.5 + 5.7 * k;
+    }
+    return general < tiles;
+}
+
 // The n products of a launch (n <= kLoraDownItems).
 static hipError_t launch_lora_mul(const LoraMulArgs& args, int n, int dt, hipStream_t s) {
-    if (args.M < kLoraTilesFrom) {
+    if (args.M * n <= kLoraRowForm) {
         bool rows = true;
         for (int i = 0; i < n; ++i)
             rows = rows && lora_row_ok(args.it[i]) &&
@@ -769,9 +798,11 @@ hipError_t launch_lora_down(const void* x, int64_t M, int64_t K, int dt, const L
     for (int i = 0; i < n; ++i) {
         const LoraMul it{x, items[i].a, items[i].u, K, items[i].r, 1, items[i].r, items[i].ldu,
                          items[i].scaling};
-        // a few rows whose factor cannot be read in 16-byte pieces, and misaligned views: the
-        // general kernel (a workgroup per row, value by value)
-        if (!lora_mul_ok(it, dt) || (M < kLoraGeneralBelow && !lora_row_ok(it))) {
+        // (a single rank of a short K: one chunk per lane is little work, and the general kernel
+        // reads it in fewer steps: 64 bf16 rows of 256 3.0 and 3.4 us, of 1024 3.7 and 3.4)
+        const bool rows = M * n <= kLoraRowForm && lora_row_ok(it) && (it.r > 1 || K >= 512);
+        if (!lora_mul_ok(it, dt) ||
+            (!rows && (M < kLoraGeneralBelow || lora_general_faster(it, M, dt)))) {
             hipError_t e;
             switch (dt) {
                 case kF32: e = lora_down_dt<kF32>(x, it.f, M, K, (int)it.r, it.scaling, it.out, it.ldo, stream); break;
