@@ -357,14 +357,13 @@ hipError_t launch_encode(const void* w, int wdt, int64_t numel, int64_t gs, uint
 // The three packers' unpack (lattice.py:386-419, 252-279, 519-533): coordinate *
 // scales.to(dtype), rounded to dtype for 2-bit and 1-bit codes.  Bound by the writes: a
 // lane writes 16 bytes (4 fp32 or 8 16-bit weights, half a code or one) of each of its
-// kDecPieces pieces, and a wave's store covers 1 KB without a gap.  One lane per 16 weights
-// left 64-byte gaps between the lanes of every store, and divided twice by the group size.
-// us for 14336 x 4096, gs 32, to fp32 / fp16 / bf16: ternary 71 / 24.5 / 29 -> 38 / 22.2 /
-// 22.7, 2-bit 71 / 24.5 / 29 -> 38 / 23 / 25, 1-bit 92 / 60 / 61 -> 39 / 24 / 24 (fp32: 6.4
-// TB/s written).
+// pieces, and a wave's store covers 1 KB without a gap.  One lane per 16 weights left 64-byte
+// gaps between the lanes of every store, and divided twice by the group size.  us for 14336 x
+// 4096, gs 32, to fp32 / fp16 / bf16: ternary 71 / 23.2 / 27.3 -> 36.4 / 20.8 / 20.9, 2-bit 70 /
+// 23.1 / 27.4 -> 36.9 / 21.3 / 22.1, 1-bit 86 / 51 / 52 -> 36.0 / 21.9 / 22.2 (fp32: 6.4 TB/s
+// written).
 
 constexpr int kDecThreads = 256;
-constexpr int kDecPieces = 4;
 
 // Bits of v in dtype ODT, rounded once (v kept a rounded fp32 product: -1 * 0 stays -0).
 template <int ODT> __device__ __forceinline__ uint32_t out_bits(float v) {
@@ -405,7 +404,7 @@ __device__ __forceinline__ void decode_run(const uint8_t* __restrict__ packed, i
                        vp = out_bits<ODT>(s);
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-            const uint32_t q = (raw * 43691u) >> 17;  // / 3, exact below 2^17
+            const uint32_t q = (raw * 43691u) >> 17;  // / 3, exact below 98304 (32-bit product)
             const uint32_t d = raw - 3u * q;
             v[i] = d == 0u ? vm : d == 1u ? vz : vp;
             raw = q;
@@ -456,23 +455,32 @@ __global__ __launch_bounds__(kDecThreads) void decode_kernel(
     }
 }
 
-// Four pieces per lane share its index work and keep four loads in flight; a tensor that
-// then leaves CUs idle takes one (512 x 512 ternary to fp16: 3.5 against 2.5 us).
+// Pieces per lane: one while that fills the chip no more than 32 times over (2M weights to
+// fp16, ternary: 3.0 us, with four pieces 3.7), then two, which share a lane's index work and keep
+// two loads in flight (1-bit 32M to fp32 24.2 and 22.8), and four for results past the last-level
+// cache (256 MB; ternary 256M to bf16 155.8 with two and 147.4).
+constexpr int64_t kDecTwoFrom = 8192, kDecFourFrom = 65536;  // blocks of one piece per lane
+
+template <int FMT, int ODT, int P>
+static hipError_t launch_decode_p(const uint8_t* packed, const uint16_t* scales, int64_t numel,
+                                  int64_t gs, int64_t runs, void* out, hipStream_t stream) {
+    const int shift = (gs & (gs - 1)) == 0 ? 63 - __builtin_clzll((unsigned long long)gs) : -1;
+    const bool vec = ((uintptr_t)out & 15u) == 0;
+    hipLaunchKernelGGL((decode_kernel<FMT, ODT, P>), dim3((unsigned)((runs + P - 1) / P)),
+                       dim3(kDecThreads), 0, stream, packed, scales, numel, gs, shift, vec, out);
+    return hipGetLastError();
+}
+
 template <int FMT, int ODT>
 static hipError_t launch_decode_t(const uint8_t* packed, const uint16_t* scales, int64_t numel,
                                   int64_t gs, void* out, hipStream_t stream) {
     constexpr int64_t kPerBlock = kDecThreads * (ODT == kF32 ? 4 : 8);
-    const int shift = (gs & (gs - 1)) == 0 ? 63 - __builtin_clzll((unsigned long long)gs) : -1;
-    const bool vec = ((uintptr_t)out & 15u) == 0;
     const int64_t runs = (numel + kPerBlock - 1) / kPerBlock;
-    if (runs >= 256 * kDecPieces)
-        hipLaunchKernelGGL((decode_kernel<FMT, ODT, kDecPieces>),
-                           dim3((unsigned)((runs + kDecPieces - 1) / kDecPieces)),
-                           dim3(kDecThreads), 0, stream, packed, scales, numel, gs, shift, vec, out);
-    else
-        hipLaunchKernelGGL((decode_kernel<FMT, ODT, 1>), dim3((unsigned)runs), dim3(kDecThreads), 0,
-                           stream, packed, scales, numel, gs, shift, vec, out);
-    return hipGetLastError();
+    if (runs < kDecTwoFrom)
+        return launch_decode_p<FMT, ODT, 1>(packed, scales, numel, gs, runs, out, stream);
+    if (runs < kDecFourFrom)
+        return launch_decode_p<FMT, ODT, 2>(packed, scales, numel, gs, runs, out, stream);
+    return launch_decode_p<FMT, ODT, 4>(packed, scales, numel, gs, runs, out, stream);
 }
 
 template <int FMT>
