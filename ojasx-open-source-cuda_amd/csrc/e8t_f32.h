@@ -16,16 +16,16 @@ template <int DT, int n> struct RawX {
     static constexpr int W = DT == kF32 ? n : n / 2;
     uint32_t w[W];
 
-    // byte offset vo; kNoRecordOffset (or any offset past the buffer) reads zeros
-    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, uint32_t vo) {
+    // byte offset vo + so (so uniform); kNoRecordOffset (or any offset past the buffer) reads zeros
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, uint32_t vo, int so = 0) {
         if constexpr (W % 4 == 0) {
 #pragma unroll
             for (int i = 0; i < W / 4; ++i) {
-                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, vo + 16u * i, 0, 0);
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, vo + 16u * i, so, 0);
                 w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
             }
         } else {
-            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(b, vo, 0, 0);
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(b, vo, so, 0);
             w[0] = v.x; w[1] = v.y;
         }
     }

@@ -117,10 +117,11 @@ __device__ __forceinline__ void lora_row(const LoraMul& it,
     const T* xr = static_cast<const T*>(it.x) + m * K;
     const T* f = static_cast<const T*>(it.f) + (KMAJOR ? 8 * sl * K : 8 * sl);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    // Two workgroups per CU need at most 128 registers: ranks over 8 take 32-bit offsets (a
-    // factor holds under 2^29 values), 118 registers.  With 64-bit ones, 131, 384 bf16 rows of
-    // K = 4096 at rank 16 took 9.0 us instead of 7.3.
-    using Off = std::conditional_t<RS == 1, int64_t, uint32_t>;
+    // Two workgroups per CU need at most 128 registers: bf16 ranks over 8 take 32-bit offsets (a
+    // factor holds under 2^29 values), 118 registers.  With 64-bit ones, 131, 384 rows of K =
+    // 4096 at rank 16 took 9.0 us instead of 7.3.  (fp16, 126 registers with 64-bit offsets, is up
+    // to 9% slower with 32-bit ones.)
+    using Off = std::conditional_t<DT == kBF16 && (RS > 1), uint32_t, int64_t>;
     // run i of chunk c: k = 8 c + i of the 8 columns, or (KMAJOR) column i of the 8 k; columns
     // past r repeat the last one, never stored
     auto load = [&](Run8<DT>& xv, Run8<DT> (&fv)[8], int64_t c) {
@@ -463,12 +464,14 @@ static bool lora_row_ok(const LoraMul& it) {
 }
 static int lora_slices(int64_t r) { return r <= 8 ? 1 : r <= 16 ? 2 : r <= 32 ? 4 : 8; }
 
-// Workgroups of the row form (one per row and product) up to which it runs: two per CU, all at
-// once.  It reads the factor from L2 once per row but has its whole K in flight; tiles of 16 rows
-// read it once per tile (us at K = 4096, rows against tiles: bf16 rank 8 512 rows 7.1 and 7.8, 640
-// rows 9.1 and 7.8; rank 64 12.9 and 13.7, 17.5 and 13.7; fp32 rank 8 12.1 and 12.6, 15.9 and
-// 12.6).
-constexpr int64_t kLoraRowForm = 512;
+// The row form runs for up to 512 rows of one product: two workgroups per CU, all at once.  It
+// reads the factor from L2 once per row but has its whole K in flight; tiles of 16 rows read it
+// once per tile (us at K = 4096, rows against tiles: bf16 rank 8 512 rows 7.1 and 7.8, 640 rows
+// 9.1 and 7.8; rank 64 12.9 and 13.7, 17.5 and 13.7; fp32 rank 8 12.1 and 12.6, 15.9 and 12.6).
+// Of several products (a backward pass forms u and v in one launch) for fewer than 512: 300
+// rows of 14336 and 4096 with rank 8 in bf16 take 14 us more in tiles, 512 rows of 4096 and
+// 4096 with rank 64 21 us less.
+static bool lora_row_form(int64_t M, int n) { return M < 512 || (M == 512 && n == 1); }
 // Rows below which a factor that cannot be read in 16-byte pieces takes the general kernel.
 constexpr int64_t kLoraGeneralBelow = 16;
 
@@ -503,7 +506,7 @@ static bool lora_general_faster(const LoraMul& it, int64_t M, int dt) {
 
 // The n products of a launch (n <= kLoraDownItems).
 static hipError_t launch_lora_mul(const LoraMulArgs& args, int n, int dt, hipStream_t s) {
-    if (args.M * n <= kLoraRowForm) {
+    if (lora_row_form(args.M, n)) {
         bool rows = true;
         for (int i = 0; i < n; ++i)
             rows = rows && lora_row_ok(args.it[i]) &&
@@ -534,14 +537,13 @@ struct LoraGradArgs {
     float* part;     // fp32 partial sums of the row splits (gridDim.y > 1)
     int64_t M, total;  // total: values per split
     int r, blocks0;  // blocks0: workgroups of it[0]
-    int span;        // groups of four rows per buffer
 };
 
 // A wave owns 128 columns c: lane (g, i) loads a[m0 + g][8 i .. 8 i + 7], eight instructions
 // of four rows each (instruction e: columns 8 i + e).  The workgroup's waves and gridDim.y
 // split the rows.  VEC: rows of a hold whole aligned groups of eight.
-// A wave walks its rows through buffers of args.span groups (offsets are 32 bits wide), so
-// any M runs with any number of row splits.
+// Every batch of rows is read through a buffer of its own (32-bit offsets, the same for all
+// batches), so any M runs with any number of row splits.
 constexpr int kLoraGradWaves = 8;
 
 template <int DT, int NT, bool VEC>
@@ -567,33 +569,49 @@ __global__ __launch_bounds__(64 * kLoraGradWaves) void lora_grad_kernel(LoraGrad
         RawX<DT, 8> a[U];
         uint32_t v[U][NT];
     };
-    // groups q .. q + U - 1 of a buffer of n groups
-    auto load = [&](Batch& f, __amdgpu_buffer_rsrc_t ar, __amdgpu_buffer_rsrc_t vr, int n, int q) {
+    // offsets of a batch's rows; rows past the wave's last lie past the buffers' ends
+    // (group u's rows of a: 4 u C values on, in the scalar offset, which the range check covers)
+    uint32_t vo_a[VEC ? 1 : 8], vo_v[U][NT];
+#pragma unroll
+    for (int e = 0; e < (VEC ? 1 : 8); ++e)
+        vo_a[e] = c0 + e < it.C ? ((uint32_t)g * (uint32_t)it.C + (uint32_t)(c0 + e)) * E
+                                : kNoRecordOffset;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int j = 16 * t + i16;
+            vo_v[u][t] = j < r ? (uint32_t)((4 * u + g) * r + j) * 4u : kNoRecordOffset;
+        }
+    const int so_a = (int)(4 * it.C * E);
+    const int64_t m_end = m_begin + 4 * count < args.M ? m_begin + 4 * count : args.M;
+    auto load = [&](Batch& f, int64_t q) {  // groups q .. q + U - 1
+        const int64_t m = m_begin + 4 * q;
+        const int rows = m < m_end ? (int)(m_end - m < 4 * U ? m_end - m : 4 * U) : 0;
+        const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(static_cast<const char*>(it.a) + m * it.C * E), (short)0,
+            (int)(rows * it.C * E), kRsrcWord3);
+        const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(it.v + m * r), (short)0, rows * r * 4, kRsrcWord3);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint32_t m = 4 * (uint32_t)(q + u) + g;
-            const uint32_t base = m * (uint32_t)it.C + (uint32_t)c0;
-            const bool live = q + u < n;
             if constexpr (VEC) {
-                f.a[u].load(ar, live && c0 < it.C ? base * E : kNoRecordOffset);
+                f.a[u].load(ar, vo_a[0], u * so_a);
             } else {
                 uint32_t w[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const uint32_t vo = live && c0 + e < it.C ? (base + e) * E : kNoRecordOffset;
                     if constexpr (DT == kF32)
-                        w[e] = __builtin_amdgcn_raw_buffer_load_b32(ar, vo, 0, 0);
+                        w[e] = __builtin_amdgcn_raw_buffer_load_b32(ar, vo_a[e], u * so_a, 0);
                     else
-                        w[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ar, vo, 0, 0);
+                        w[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ar, vo_a[e],
+                                                                              u * so_a, 0);
                 }
                 f.a[u].set(w);
             }
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const int j = 16 * t + i16;
-                f.v[u][t] = __builtin_amdgcn_raw_buffer_load_b32(
-                    vr, live && j < r ? (m * r + j) * 4u : kNoRecordOffset, 0, 0);
-            }
+            for (int t = 0; t < NT; ++t)
+                f.v[u][t] = __builtin_amdgcn_raw_buffer_load_b32(vr, vo_v[u][t], 0, 0);
         }
     };
     f32x4 acc[8][NT];
@@ -610,26 +628,15 @@ __global__ __launch_bounds__(64 * kLoraGradWaves) void lora_grad_kernel(LoraGrad
                 for (int t = 0; t < NT; ++t)
                     acc[e][t] = mfma4(f.a[u].get(e), __uint_as_float(f.v[u][t]), acc[e][t]);
     };
-    for (int64_t q0 = 0; q0 < count; q0 += args.span) {
-        // rows past the buffer's last belong to others or lie past the end
-        const int n = (int)(count - q0 < args.span ? count - q0 : args.span);
-        const int64_t m0 = m_begin + 4 * q0;
-        const int64_t left = args.M - m0 < 4 * n ? args.M - m0 : 4 * n;
-        const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(static_cast<const char*>(it.a) + m0 * it.C * E), (short)0,
-            (int)(left * it.C * E), kRsrcWord3);
-        const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(it.v + m0 * r), (short)0, (int)(left * r * 4), kRsrcWord3);
-        Batch f0, f1;
-        load(f0, ar, vr, n, 0);
-        for (int q = 0; q < n; q += 2 * U) {
-            load(f1, ar, vr, n, q + U);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(f0);
-            load(f0, ar, vr, n, q + 2 * U);
-            __builtin_amdgcn_sched_barrier(0);
-            if (q + U < n) compute(f1);
-        }
+    Batch f0, f1;
+    load(f0, 0);
+    for (int64_t q = 0; q < count; q += 2 * U) {
+        load(f1, q + U);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(f0);
+        load(f0, q + 2 * U);
+        __builtin_amdgcn_sched_barrier(0);
+        if (q + U < count) compute(f1);
     }
 #pragma unroll
     for (int h = kLoraGradWaves / 2; h >= 1; h /= 2) {
@@ -686,13 +693,6 @@ static int64_t lora_grad_splits(int64_t M, int64_t blocks) {
     return s < 1 ? 1 : s;
 }
 
-// Groups of four rows per buffer: 256 MB of fp32 rows (refilling the pipeline that often costs
-// nothing), at least one trip of the loop, which at widths under kLoraGradMaxWidth is 1 GB.
-static int lora_grad_span(int64_t cmax) {
-    const int64_t n = (1ll << 28) / (cmax * 16) / 8 * 8;
-    return n < 8 ? 8 : (int)n;
-}
-
 static int64_t lora_blocks(int64_t C) { return (C + 127) / 128; }
 
 size_t lora_grads_bytes(int64_t M, int64_t N, int64_t K, int64_t r, bool need_a, bool need_b) {
@@ -745,8 +745,6 @@ hipError_t launch_lora_grads(const void* x, const void* gy, const float* u, cons
     args.part = part;
     args.M = M;
     args.r = (int)r;
-    const int64_t cmax = K > N ? K : N;
-    args.span = lora_grad_span(cmax > kLoraMaxRank ? cmax : kLoraMaxRank);
     int64_t splits = lora_grad_splits(M, blocks);
     const int64_t fit = part ? (int64_t)(part_bytes / ((size_t)args.total * 4)) : 0;
     if (splits > fit) splits = fit < 2 ? 1 : fit;
@@ -800,7 +798,7 @@ hipError_t launch_lora_down(const void* x, int64_t M, int64_t K, int dt, const L
                          items[i].scaling};
         // (a single rank of a short K: one chunk per lane is little work, and the general kernel
         // reads it in fewer steps: 64 bf16 rows of 256 3.0 and 3.4 us, of 1024 3.7 and 3.4)
-        const bool rows = M * n <= kLoraRowForm && lora_row_ok(it) && (it.r > 1 || K >= 512);
+        const bool rows = lora_row_form(M, n) && lora_row_ok(it) && (it.r > 1 || K >= 512);
         if (!lora_mul_ok(it, dt) ||
             (!rows && (M < kLoraGeneralBelow || lora_general_faster(it, M, dt)))) {
             hipError_t e;

@@ -69,8 +69,8 @@ def test_many_rows(M, N_out, K):
 
 
 @pytest.mark.parametrize("M,N_out,K,r,dtype", [
-    (80007, 16384, 64, 20, bf16),  # a wave's rows in two and a half buffers
-    (9001, 2500, 80, 33, f16),     # and in one, by single values
+    (80007, 16384, 64, 20, bf16),
+    (9001, 2500, 80, 33, f16),  # by single values
 ])
 def test_without_workspace(M, N_out, K, r, dtype):
     x, gy, a, b, pk, sc = _operands(M, N_out, K, r, dtype)
