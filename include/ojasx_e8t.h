@@ -96,7 +96,8 @@ int ojx_gemm_workspace_bytes(int fmt, int bwd, int64_t M, int64_t N, int64_t K, 
  *   x, y, bias in `dtype`; bias may be NULL.  Wdeq follows the decoder's rule for `dtype`.
  *   Any K >= 1 (flat layout).  F16/BF16 with K % 256 == 0, gs in {16, 32, 64} and M <= 16
  *   run an MFMA decode GEMV; F16/BF16 with K % 64 == 0, gs in {16, 32, 64} and M > 16 the
- *   MFMA prefill GEMM; other shapes and F32 use a general tiled kernel.  Never declines.
+ *   MFMA prefill GEMM; other shapes and F32 the fp32 matrix instruction where rows hold whole
+ *   scale groups of a power of two, else a general tiled kernel.  Never declines.
  *   workspace: 16-byte aligned device scratch of workspace_bytes (NULL with 0 allowed),
  *   see ojx_gemm_workspace_bytes. */
 int ojx_e8t_gemm_fwd(const void* x, const uint8_t* packed, const uint16_t* scales,

@@ -17,9 +17,11 @@
 // Decoded weights follow the reference's dtype rule (coord * scales.to(dtype), rounded to
 // dtype for 2-bit and 1-bit codes); products and sums are fp32.
 //
-// Bound: the 8 matrix instructions of 32 cycles per 512 weights and 16 activation rows (12.5 us
-// for M = 16 of 14336 x 4096) and the decode's 20-30 VALU per code, which share a SIMD's issue
-// slots, plus the first loads' round trip in short launches.  Rows are split over the
+// Bound: loads' round trips in launches of one or two workgroups per CU (22 to 43% of the wave
+// cycles wait), beside the 8 matrix instructions of 32 cycles per 512 weights and 16 activation
+// rows (12.5 us for M = 16 of 14336 x 4096, 34 to 37% of the cycles) and the decode's 20-30 VALU
+// per code (17%).  The backward also reads its codes 6.5 times: a workgroup's 128 columns take 24
+// bytes of each 128-byte line.  Rows are split over the
 // workgroup's waves (LDS reduction), the backward's also over workgroups (fp32 partial sums
 // in the caller's workspace), since one 16-row tile is a long serial chain of little work.
 // Measured against the 64 x 64 SIMT tiles of e8t_gemm_generic.hip (which decode every weight

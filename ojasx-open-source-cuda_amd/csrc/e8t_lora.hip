@@ -1,11 +1,17 @@
-// e8t_lora.hip -- down-projection of a LoRA adapter for the fused E8 forwards.
+// e8t_lora.hip -- down-projections and gradients of a LoRA adapter.
 //
 // E8LatticeLinear.forward adds scaling * ((x @ A) @ B) to the E8 op's output
 // (ojasx2/math/lattice.py:839-842; A [in, r], B [r, out]).  The fused forwards of this
 // library add u @ B inside their output epilogue (before the one rounding to the activation
-// dtype), with u = scaling * (x @ A) in fp32 [M, r] computed here.  The general kernel takes
-// any dtype, K and r: one workgroup per activation row, the 256 threads splitting K, r
-// partial sums per thread reduced across the wave by shuffles and across the waves in LDS.
+// dtype), with u = scaling * (x @ A) in fp32 [M, r] computed here; the backward forms v =
+// scaling * (gy @ B^T) with the same kernels, adds v @ A^T in the dX epilogue and computes A's
+// and B's gradients from v and u here.
+//
+// Three forms of the down-projection: lora_row_kernel (a workgroup per row, 16-byte loads; up to
+// 512 rows), lora_mul_kernel (tiles of 16 rows on the matrix unit) and lora_down_kernel, the
+// general one: any dtype, K and r, one workgroup per activation row, the 256 threads splitting
+// K value by value, r partial sums per thread reduced across the wave by shuffles and across
+// the waves in LDS.
 
 #include <hip/hip_runtime.h>
 
