@@ -69,4 +69,4 @@ def test_time_grows_with_the_size(op):
             torch.cuda.synchronize()
             best[i] = min(best[i], a.elapsed_time(b))
     print(f"decode {op} {best}", flush=True)
-    assert best[1] < 1.2 * best[0]  # 1.1; 1.28 to 1.4 with four pieces per lane for the larger
+    assert best[1] < 1.24 * best[0]  # 1.1; 1.28 to 1.4 with four pieces per lane for the larger

@@ -45,4 +45,4 @@ def test_types_agree(bwd, code_bytes, gs):
     us = [_us(lambda: bwd(gy, packed, scales, N, K, gs))
           for gy in (torch.zeros(M, N, dtype=t, device=DEV) for t in (torch.bfloat16, torch.float16))]
     print(f"bwd gs={gs} {us}", flush=True)
-    assert max(us) < 1.3 * min(us)
+    assert max(us) < 1.4 * min(us)  # 1.1 to 1.2; 1.6 with the waits
